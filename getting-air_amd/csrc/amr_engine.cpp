@@ -732,7 +732,12 @@ int macro_step(lbm_amr* a) {
     const int n = deep ? a->deep.back().nactive : a->nactive;
     HIPCHK(launch_pool_force(d.q, deep ? a->deep.back().pool[0] : a->pool[0], G,
                              deep ? a->deep.back().active : a->active, n, a->force_partials, a->stream));
-    ForceFinalizeArgs fa{a->force_partials, pool_force_blocks(d.rb, n), a->history, a->written, kForceCap};
+    ForceSum fa{};
+    fa.partials[0] = a->force_partials;
+    fa.nslots = pool_force_blocks(d.rb, n);
+    fa.history = a->history;
+    fa.written = a->written;
+    fa.capacity = kForceCap;
     HIPCHK(launch_force_finalize(fa, a->stream));
   }
   const ParentRef P0 = dense_parent(a, l0);

@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <vector>
 
 namespace lbm {
 
@@ -49,6 +50,28 @@ __host__ __device__ inline size_t lat_elem(int q, int i, uint32_t c) {
   return ((size_t)(c / kLatBlock) * q + i) * kLatBlock + c % kLatBlock;
 }
 
+// Force partials of a launch and where their sums go: slots summed in slot
+// order, one record [fx, fy, fz, tx, ty, tz] per step appended to the history
+// ring.
+struct ForceSum {
+  const double* partials[2];    // the launch's first step and, if it took two, its second (else null):
+                                // per slot [3] (force) with `cells`, else [6] (force and torque)
+  uint32_t nslots;
+  const uint32_t* cells;        // per slot its boundary cell, or null
+  double centre[3];             // torque arm origin
+  int32_t nx, ny, periodic_arm; // 2D: nearest periodic image for the arm
+  InvariantDiv div_nx, div_ny;
+  double* history;
+  unsigned long long* written;  // records written since reset
+  uint32_t capacity;
+};
+// Ranks of the boundary cells (ascending cell index) among each 64 cells: a
+// boundary cell's slot is base + the number of mask bits below its own.
+struct BoundaryRank {
+  uint64_t mask;
+  uint32_t base, pad;
+};
+
 // Everything one fused stream-collide launch needs besides the two lattices.
 struct StepArgs {
   int32_t nx, ny, nz;
@@ -87,19 +110,20 @@ struct StepArgs {
   // (coveredByFiner, common_d3_step.wgsl:104-114).  Null without AMR.
   const int32_t* cover;
   int32_t cover_rb, cover_nbx, cover_nby;
-  // Momentum-exchange force, fused into the step: tiles holding a fluid cell
-  // with a solid streaming source own a slot of 6 FP64 partials.
-  const int32_t* force_slot;  // per logical tile: slot index or -1; null: no force
-  double* force_partials;     // [slot][6] of this step (lattice parity buffer)
-  // The previous step's partials are summed by the first wave of block 0 of
-  // this launch (in the same fixed order as k_force_finalize), so a run of
-  // steps needs no separate reduction launch per step.
+  // Momentum-exchange force, fused into the step.  Bounce-back: every
+  // boundary cell (a fluid cell with a solid streaming source) leaves its
+  // force in a slot of its own, so the record, summed in cell order, does not
+  // depend on how a kernel cuts the grid.  The diffuse coupling's force cells
+  // fill a band around the body: there each tile holding one has a slot of 6
+  // partials (force_slot: per logical tile, its slot or -1).
+  const BoundaryRank* boundary;  // bounce-back: per 64 cells; null: no force
+  const int32_t* force_slot;     // diffuse: per tile; null: no force
+  double* force_partials;        // this step's slots (lattice parity buffer)
+  // The previous step's slots are summed by block 0 of this launch (in the
+  // same fixed order as k_force_finalize), so a run of steps needs no separate
+  // reduction launch per step.
   int32_t finalize_prev;
-  const double* prev_partials;
-  uint32_t nslots;
-  double* history;
-  unsigned long long* written;
-  uint32_t hist_cap;
+  ForceSum prev;
   double body_c[3];           // torque arm origin
   int32_t periodic_arm;       // 2D: nearest periodic image for the arm
   // The diffuse penalty coupling of the pinned body (the DIFF kernels, in
@@ -142,16 +166,6 @@ struct BatchArgs {
   const BatchSolve* solves;
   const BatchTile* tiles;
   int32_t launch;        // index of this launch within the chunk
-};
-
-// Sums the force partial slots in slot order and appends one record
-// [fx, fy, fz, tx, ty, tz] to the history ring.
-struct ForceFinalizeArgs {
-  const double* partials;
-  uint32_t nslots;
-  double* history;
-  unsigned long long* written;  // records written since reset
-  uint32_t capacity;
 };
 
 struct TotalsArgs {
@@ -197,9 +211,44 @@ struct PersistBarrier {
 hipError_t launch_step_persistent(int q, int storage, bool general, bool nontemporal, int occ, bool rows, bool force,
                                   const BatchArgs& b, uint32_t ntiles, int bx, int by, int steps, PersistBarrier* bar,
                                   hipStream_t s);
+// The launches above for one lattice (dense_step.h); persistent_steps <= 0: one
+// batched launch.
+template <int Q>
+struct DenseStep {
+  static hipError_t step(int storage, bool general, bool nt, int occ, const void* fin, void* fout, const StepArgs& a,
+                         int bx, int by, hipStream_t s, bool diffuse);
+  static hipError_t batch(int storage, bool general, bool nt, int occ, bool rows, bool force, const BatchArgs& b,
+                          uint32_t ntiles, int bx, int by, int persistent_steps, PersistBarrier* bar, hipStream_t s);
+};
+// LDS share of a block of `threads` under the cap (0: none).
+size_t occ_share(int occ, int threads);
 // Whether `occ` waves per SIMD can be set exactly for blocks of `threads`.
 bool occupancy_cap_ok(int occ, int threads);
-hipError_t launch_force_finalize(const ForceFinalizeArgs& a, hipStream_t s);
+// Two steps in one launch (dense_pair.hip), fp32 3D lattices on the bounce-back
+// coupling without a moving body: gout holds the state two steps after gin.
+// A block marches a column of 64 x rows cells through some planes along z,
+// keeping the step in between in LDS.
+struct PairBlock {
+  int32_t x0, y0, z0, planes;  // the column's first cell, its planes
+};
+struct PairPlan {
+  int32_t rows = 0;                 // rows of a block's column (0: no pair launches)
+  std::vector<PairBlock> blocks;
+};
+struct PairArgs {
+  const PairBlock* blocks;
+  uint32_t nblocks;
+  int32_t rows;
+  double* force2;         // second step's force slots (StepArgs::force_partials: the first's)
+  int32_t finalize_prev;  // block 0 appends the previous launch's records (StepArgs::prev)
+};
+// The blocks for a grid whose boundary cells (ascending) are given; rows 0
+// where one-step launches are the faster ones or the pair kernel does not
+// take the grid.
+PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary);
+hipError_t launch_step_pair(int q, bool general, const void* fin, void* fout, const StepArgs& a, const PairArgs& p,
+                            hipStream_t s);
+hipError_t launch_force_finalize(const ForceSum& a, hipStream_t s);
 hipError_t launch_totals(int q, int storage, const void* f, const TotalsArgs& a, int nblocks, hipStream_t s);
 // The wire format is plane-major f ([Q][ncells] float); the lattice uses the
 // block layout below.

@@ -99,9 +99,15 @@ struct lbm_solve {
   uint8_t* cls = nullptr;
   uint32_t* links = nullptr;        // bounce-back link masks of the cells next to the body
   std::vector<uint32_t> boundary;   // fluid cells with a solid streaming source
-  int32_t* force_slot = nullptr;    // per tile of the current shape
+  // Force slots.  Bounce-back: one per boundary cell, found through the cells'
+  // ranks; two sets per lattice parity where a launch may take two steps.
+  // Diffuse: one per tile of the current shape that holds a force cell.
+  BoundaryRank* ranks = nullptr;
+  uint32_t* boundary_cells = nullptr;
+  int32_t* force_slot = nullptr;
   double* force_partials = nullptr;
   uint32_t nslots = 0;
+  size_t rank_bytes = 0, cell_bytes = 0;
   int slot_bx = 0, slot_by = 0, slot_lin = -1;
   size_t slot_bytes = 0, partial_bytes = 0;
   double* scratch = nullptr;        // totals partials
@@ -120,13 +126,16 @@ struct lbm_solve {
   int bx = 64, by = 1, swz = 1, nt = 0;
   int occ = 0;                      // waves-per-SIMD cap of the step launches (0: none)
   int lin = 0;                      // linear tiles (blocks of consecutive cells)
-  bool force_pending = false;       // last step's force partials not yet summed
+  int force_pending = 0;            // steps of the last launch whose forces are not yet summed
+  int pair_rows = 0;                // two-step launches: rows of a block (0: none),
+  PairBlock* pair_blocks = nullptr; // and the blocks
+  uint32_t pair_nblocks = 0;
   bool tuned = false;
   bool initialised = false;
   long long step = 0;
   size_t bytes = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
-  int graph_bx = 0, graph_by = 0, graph_swz = 0, graph_nt = 0, graph_occ = 0, graph_lin = 0;
+  int graph_bx = 0, graph_by = 0, graph_swz = 0, graph_nt = 0, graph_occ = 0, graph_lin = 0, graph_pair = 0;
   Arena* arena = nullptr;           // pool the buffers come from (serve loop), or null
   bool own_stream = true;
   // Both parity graphs and the autotuned tile are made when the state is set
@@ -222,6 +231,33 @@ void pair_constants(StepArgs& a, const lbm_desc& d) {
 // CHI_EPS of the diffuse coupling (main-3d.js:1026 default 1.5).
 float chi_eps(const lbm_desc& d) { return d.chi_eps > 0.f ? d.chi_eps : 1.5f; }
 
+// Force slots of step `sub` (0, or 1: the second step of a two-step launch)
+// of a launch that read lattice `parity`.
+double* force_set(const lbm_solve* s, int parity, int sub) {
+  const size_t width = s->d.diffuse ? 6 : 3, subs = s->arena ? 1 : 2;
+  return s->force_partials + (size_t)s->nslots * width * (parity * subs + sub);
+}
+// The sum of the forces of a launch of `steps` steps that read lattice `parity`.
+ForceSum force_sum(const lbm_solve* s, int parity, int steps) {
+  ForceSum f{};
+  f.partials[0] = force_set(s, parity, 0);
+  f.partials[1] = steps > 1 ? force_set(s, parity, 1) : nullptr;
+  f.nslots = s->nslots;
+  f.cells = s->d.diffuse ? nullptr : s->boundary_cells;
+  f.centre[0] = s->d.body.centre[0];
+  f.centre[1] = s->d.body.centre[1];
+  f.centre[2] = s->dim == 3 ? s->d.body.centre[2] : 0.0;
+  f.nx = s->d.nx;
+  f.ny = s->d.ny;
+  f.periodic_arm = s->dim == 2;
+  f.div_nx = make_invariant_div((uint32_t)s->d.nx);
+  f.div_ny = make_invariant_div((uint32_t)s->d.ny);
+  f.history = s->history;
+  f.written = s->written;
+  f.capacity = kHistoryCap;
+  return f;
+}
+
 StepArgs step_args(lbm_solve* s, bool write_mac, bool with_force) {
   StepArgs a{};
   const lbm_desc& d = s->d;
@@ -248,14 +284,10 @@ StepArgs step_args(lbm_solve* s, bool write_mac, bool with_force) {
   a.salt_out = s->salt + (1 - s->parity);
   if (with_force && s->body && s->nslots) {
     // partial buffers alternate with the lattice parity
-    const size_t stride = (size_t)s->nslots * 6;
-    a.force_slot = s->force_slot;
-    a.force_partials = s->force_partials + stride * s->parity;
-    a.prev_partials = s->force_partials + stride * (1 - s->parity);
-    a.nslots = s->nslots;
-    a.history = s->history;
-    a.written = s->written;
-    a.hist_cap = kHistoryCap;
+    if (d.diffuse) a.force_slot = s->force_slot;
+    else a.boundary = s->ranks;
+    a.force_partials = force_set(s, s->parity, 0);
+    a.prev = force_sum(s, 1 - s->parity, 1);
   }
   a.body_c[0] = d.body.centre[0];
   a.body_c[1] = d.body.centre[1];
@@ -285,10 +317,50 @@ StepArgs step_args(lbm_solve* s, bool write_mac, bool with_force) {
   return a;
 }
 
-// Maps every tile of the current shape that holds a boundary cell to a slot,
-// in ascending tile order (so the finalize sum order is fixed per shape).
+// Bounce-back: every boundary cell's slot is its rank in ascending cell
+// order, the same for every tile shape and kernel.
+int build_boundary_slots(lbm_solve* s) {
+  const size_t groups = (s->N + 63) / 64;
+  std::vector<BoundaryRank> rank(groups, BoundaryRank{0, 0, 0});
+  for (uint32_t cell : s->boundary) rank[cell / 64].mask |= 1ull << (cell % 64);
+  uint32_t n = 0;
+  for (BoundaryRank& r : rank) {
+    r.base = n;
+    n += (uint32_t)__builtin_popcountll(r.mask);
+  }
+  s->rank_bytes = groups * sizeof(BoundaryRank);
+  s->cell_bytes = std::max<size_t>(n, 1) * 4;
+  // one set per lattice parity and step of a launch (one step in a pool)
+  s->partial_bytes = (size_t)(s->arena ? 2 : 4) * std::max<size_t>(n, 1) * 3 * 8;
+  int rc = dalloc(s, &s->ranks, s->rank_bytes);
+  if (!rc) rc = dalloc(s, &s->boundary_cells, s->cell_bytes);
+  if (!rc) rc = dalloc(s, &s->force_partials, s->partial_bytes);
+  if (rc) return rc;
+  HIPCHK(hipMemcpyAsync(s->ranks, rank.data(), s->rank_bytes, hipMemcpyHostToDevice, s->stream));
+  if (n) HIPCHK(hipMemcpyAsync(s->boundary_cells, s->boundary.data(), (size_t)n * 4, hipMemcpyHostToDevice, s->stream));
+  HIPCHK(hipStreamSynchronize(s->stream));
+  s->nslots = n;
+  return LBM_OK;
+}
+
+// The two-step launch's blocks, where pairs are the faster form.
+int build_pair_blocks(lbm_solve* s) {
+  const PairPlan plan = pair_plan(s->q, s->storage, s->general, s->d.nx, s->d.ny, s->d.nz, s->boundary);
+  if (plan.rows <= 0) return LBM_OK;
+  const size_t bytes = plan.blocks.size() * sizeof(PairBlock);
+  int rc = dalloc(s, &s->pair_blocks, bytes);
+  if (rc) return rc;
+  HIPCHK(hipMemcpyAsync(s->pair_blocks, plan.blocks.data(), bytes, hipMemcpyHostToDevice, s->stream));
+  HIPCHK(hipStreamSynchronize(s->stream));
+  s->pair_rows = plan.rows;
+  s->pair_nblocks = (uint32_t)plan.blocks.size();
+  return LBM_OK;
+}
+
+// Diffuse: maps every tile of the current shape that holds a force cell to a
+// slot, in ascending tile order (so the finalize sum order is fixed per shape).
 int build_force_slots(lbm_solve* s) {
-  if (!s->body) return LBM_OK;
+  if (!s->body || !s->d.diffuse) return LBM_OK;
   if (s->slot_bx == s->bx && s->slot_by == s->by && s->slot_lin == s->lin && s->force_slot) return LBM_OK;
   const lbm_desc& d = s->d;
   const int ntx = (d.nx + s->bx - 1) / s->bx, nty = (d.ny + s->by - 1) / s->by;
@@ -308,7 +380,7 @@ int build_force_slots(lbm_solve* s) {
   s->force_slot = nullptr;
   s->force_partials = nullptr;
   s->slot_bytes = ntiles * 4;
-  s->partial_bytes = 2 * std::max<size_t>(n, 1) * 6 * 8;  // one set per lattice parity
+  s->partial_bytes = 2 * 2 * std::max<size_t>(n, 1) * 6 * 8;  // as force_set lays them out
   int rc = dalloc(s, &s->force_slot, s->slot_bytes);
   if (rc) return rc;
   rc = dalloc(s, &s->force_partials, s->partial_bytes);
@@ -335,24 +407,46 @@ int enqueue_step(lbm_solve* s, bool write_mac, bool finalize_prev) {
     if (e != hipSuccess) return hip_fail(e, "rigid body launch");
   }
   StepArgs a = step_args(s, write_mac, true);
-  a.finalize_prev = finalize_prev && a.force_slot ? 1 : 0;
+  const bool force = a.boundary || a.force_slot;
+  a.finalize_prev = finalize_prev && force ? 1 : 0;
+  a.prev = force ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
   hipError_t e = launch_step(s->q, s->storage, s->general, s->nt, s->occ, fin, fout, a, s->bx, s->by, s->stream,
                              s->d.diffuse != 0);
   if (e != hipSuccess) return hip_fail(e, "step kernel launch");
-  s->force_pending = a.force_slot != nullptr;
+  s->force_pending = force ? 1 : 0;
   s->parity ^= 1;
   s->step++;
   return LBM_OK;
 }
 
-// Appends the force record of the last enqueued step.
+// Two steps in one launch; the lattice parity flips once.
+int enqueue_pair(lbm_solve* s, bool write_mac, bool finalize_prev) {
+  StepArgs a = step_args(s, write_mac, true);
+  a.finalize_prev = finalize_prev && a.boundary ? 1 : 0;
+  a.prev = a.boundary ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
+  PairArgs p{};
+  p.blocks = s->pair_blocks;
+  p.nblocks = s->pair_nblocks;
+  p.rows = s->pair_rows;
+  p.force2 = a.boundary ? force_set(s, s->parity, 1) : nullptr;
+  p.finalize_prev = a.finalize_prev;
+  hipError_t e = launch_step_pair(s->q, s->general, s->f[s->parity], s->f[1 - s->parity], a, p, s->stream);
+  if (e != hipSuccess) return hip_fail(e, "two-step kernel launch");
+  s->force_pending = a.boundary ? 2 : 0;
+  s->parity ^= 1;
+  s->step += 2;
+  return LBM_OK;
+}
+
+// Whether this solve's steps may go in pairs now.
+bool pairs_on(const lbm_solve* s) { return s->pair_rows > 0 && !s->rigid; }
+
+// Appends the force records of the last enqueued launch.
 int flush_force(lbm_solve* s) {
   if (!s->force_pending) return LBM_OK;
-  ForceFinalizeArgs fa{s->force_partials + (size_t)s->nslots * 6 * (1 - s->parity), s->nslots, s->history,
-                       s->written, kHistoryCap};
-  hipError_t e = launch_force_finalize(fa, s->stream);
+  hipError_t e = launch_force_finalize(force_sum(s, 1 - s->parity, s->force_pending), s->stream);
   if (e != hipSuccess) return hip_fail(e, "force finalize launch");
-  s->force_pending = false;
+  s->force_pending = 0;
   return LBM_OK;
 }
 
@@ -393,15 +487,23 @@ void drop_graphs(lbm_solve* s) {
   }
 }
 
-// Captures kGraphChunk steps starting at the current parity.
+// Captures kGraphChunk steps starting at the current parity (an even number of
+// launches, also in pairs, so the parity returns).
 int build_graph(lbm_solve* s) {
   const int p = s->parity;
   hipGraph_t g = nullptr;
   HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
   const long long step0 = s->step;
-  const bool pending0 = s->force_pending;
+  const int pending0 = s->force_pending;
+  const bool pairs = pairs_on(s);
+  // a chunk follows a launch of its own kind (lbm_step)
+  s->force_pending = s->body && s->nslots ? (pairs ? 2 : 1) : 0;
   int rc = LBM_OK;
-  for (int k = 0; k < kGraphChunk && rc == LBM_OK; k++) rc = enqueue_step(s, false, true);
+  if (pairs) {
+    for (int k = 0; k < kGraphChunk / 2 && rc == LBM_OK; k++) rc = enqueue_pair(s, false, true);
+  } else {
+    for (int k = 0; k < kGraphChunk && rc == LBM_OK; k++) rc = enqueue_step(s, false, true);
+  }
   hipError_t e = hipStreamEndCapture(s->stream, &g);
   s->step = step0;
   s->parity = p;
@@ -416,7 +518,14 @@ int build_graph(lbm_solve* s) {
   if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
   s->graph_bx = s->bx; s->graph_by = s->by; s->graph_swz = s->swz; s->graph_nt = s->nt; s->graph_occ = s->occ;
   s->graph_lin = s->lin;
+  s->graph_pair = pairs;
   return LBM_OK;
+}
+
+// Whether the captured chunks are of the current tile and launch form.
+bool graphs_current(const lbm_solve* s) {
+  return s->graph_bx == s->bx && s->graph_by == s->by && s->graph_swz == s->swz && s->graph_nt == s->nt &&
+         s->graph_occ == s->occ && s->graph_lin == s->lin && s->graph_pair == (int)pairs_on(s);
 }
 
 int autotune(lbm_solve* s);
@@ -430,9 +539,7 @@ int prepare_graphs(lbm_solve* s) {
     int rc = autotune(s);
     if (rc) return rc;
   }
-  if (s->graph_bx != s->bx || s->graph_by != s->by || s->graph_swz != s->swz || s->graph_nt != s->nt ||
-      s->graph_occ != s->occ || s->graph_lin != s->lin)
-    drop_graphs(s);
+  if (!graphs_current(s)) drop_graphs(s);
   const int p0 = s->parity;
   for (int p = 0; p < 2; p++) {
     if (s->graph[p]) continue;
@@ -559,14 +666,14 @@ int build_boundary(lbm_solve* s) {
           }
         }
       }
-  return build_force_slots(s);
+  return d.diffuse ? build_force_slots(s) : build_boundary_slots(s);
 }
 
 void release(lbm_solve* s) {
   if (!s) return;
   drop_graphs(s);
-  void* ptrs[] = {s->f[0], s->f[1], s->mac, s->cls, s->links, s->force_slot, s->force_partials, s->scratch,
-                  s->counters, s->history, s->written, s->totals, s->salt};
+  void* ptrs[] = {s->f[0], s->f[1], s->mac, s->cls, s->links, s->ranks, s->boundary_cells, s->pair_blocks, s->force_slot,
+                  s->force_partials, s->scratch, s->counters, s->history, s->written, s->totals, s->salt};
   for (void* p : ptrs) {
     if (!p) continue;
     if (s->arena) s->arena->release(p);
@@ -581,7 +688,7 @@ void release(lbm_solve* s) {
 }
 
 int reset_history(lbm_solve* s) {
-  s->force_pending = false;
+  s->force_pending = 0;
   HIPCHK(hipMemsetAsync(s->written, 0, sizeof(unsigned long long), s->stream));
   return LBM_OK;
 }
@@ -656,6 +763,10 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
       return rc;
     }
   }
+  if (!arena && !desc->diffuse && (rc = build_pair_blocks(s))) {
+    release(s);
+    return rc;
+  }
   if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) {
     release(s);
     return hip_fail(e, "hipStreamSynchronize");
@@ -700,10 +811,21 @@ size_t solve_footprint(const lbm_desc* d) {
   size_t total = 2 * al(lattice_elems(d->q, (uint32_t)n) * elem) + al(n * 16) + al((size_t)kTotalsBlocks * 4 * 8) + al(64) +
                  al((size_t)kHistoryCap * 6 * 8) + al(8) + al(64) + al(8);
   if (d->body.shape != LBM_BODY_NONE) {
-    // class bytes, link masks, one slot index per tile (tiles of at least 64
-    // cells) and two parity sets of 6 partials per slot (at most one per tile)
+    // class bytes, link masks; the boundary cells' ranks, indices and two
+    // parity sets of 3 partials.  A boundary cell's centre lies less than a
+    // link from the surface (sqrt 3, in 2D sqrt 2), so the unit cells around
+    // them lie in that shell grown by half a cell's diagonal, whose volume
+    // bounds their number; and never less than a slot index per tile of 64
+    // cells and two sets of 6 partials per tile.
+    const bool d3 = d->q != 9;
+    const double half = d3 ? 0.8661 : 0.7072, r1 = (double)d->body.radius + 3.0 * half,
+                 r0 = std::max(0.0, (double)d->body.radius - half), pi = 3.14159265358979;
+    const double shell = d3 ? 4.0 / 3.0 * pi * (r1 * r1 * r1 - r0 * r0 * r0) : pi * (r1 * r1 - r0 * r0);
+    const size_t cells = (size_t)std::min((double)n, shell + 1.0);
     const size_t tiles = (n + 63) / 64 + d->ny * (d->q == 9 ? 1 : d->nz);
-    total += al(n) + al(n * 4) + al(tiles * 4) + al(2 * tiles * 6 * 8);
+    total += al(n) + al(n * 4) +
+             std::max(al((n + 63) / 64 * sizeof(BoundaryRank)) + al(cells * 4) + al(2 * cells * 3 * 8),
+                      al(tiles * 4) + al(2 * tiles * 6 * 8));
   }
   return total;
 }
@@ -746,13 +868,7 @@ int solve_advance(lbm_solve* s, int steps, bool finalize_force) {
   s->parity ^= steps & 1;
   if (finalize_force && s->body && s->nslots) {
     // the partials of the last step live in the buffer of the parity it read
-    ForceFinalizeArgs fa{};
-    fa.partials = s->force_partials + (size_t)s->nslots * 6 * (1 - s->parity);
-    fa.nslots = s->nslots;
-    fa.history = s->history;
-    fa.written = s->written;
-    fa.capacity = kHistoryCap;
-    HIPCHK(launch_force_finalize(fa, s->stream));
+    HIPCHK(launch_force_finalize(force_sum(s, 1 - s->parity, 1), s->stream));
   }
   s->initialised = true;
   return LBM_OK;
@@ -914,7 +1030,7 @@ int lbm_load_state(lbm_solve* s, const void* buf, size_t bytes) {
   s->salt0 = h.salt;
   s->step_at_salt0 = h.step;
   s->initialised = true;
-  s->force_pending = false;
+  s->force_pending = 0;
   rc = reset_history(s);
   if (rc) return rc;
   return prepare_graphs(s);
@@ -942,13 +1058,34 @@ int lbm_step(lbm_solve* s, int32_t n) {
     int rc = autotune(s);
     if (rc) return rc;
   }
-  if (s->graph_bx != s->bx || s->graph_by != s->by || s->graph_swz != s->swz || s->graph_nt != s->nt ||
-      s->graph_occ != s->occ || s->graph_lin != s->lin)
-    drop_graphs(s);
+  if (!graphs_current(s)) drop_graphs(s);
+  int rc = LBM_OK;
+  if (pairs_on(s)) {
+    // An odd step first, then pairs: one eagerly (so that every chunk follows
+    // a pair, whose forces its first launch sums), captured chunks, single
+    // pairs, the last of them writing the macroscopic field.
+    if (n & 1) rc = enqueue_step(s, n == 1, false);
+    int left = n / 2;
+    bool first = true;
+    while (left > 0 && rc == LBM_OK) {
+      if (!first && left > kGraphChunk / 2) {
+        if (!s->graph[s->parity] && (rc = build_graph(s))) return rc;
+        HIPCHK(hipGraphLaunch(s->graph[s->parity], s->stream));
+        s->step += kGraphChunk;
+        left -= kGraphChunk / 2;
+        continue;
+      }
+      rc = enqueue_pair(s, left == 1, s->force_pending != 0);
+      first = false;
+      left--;
+    }
+    if (rc) return rc;
+    return flush_force(s);
+  }
   // First step eagerly (nothing earlier in this call to finalize), then
   // captured chunks and single steps that each finalize their predecessor's
   // force, the last step writing the macroscopic field, then the last force.
-  int rc = enqueue_step(s, n == 1, false);
+  rc = enqueue_step(s, n == 1, false);
   if (rc) return rc;
   int left = n - 2;  // steps between the first and the last
   while (left >= kGraphChunk) {
@@ -959,7 +1096,6 @@ int lbm_step(lbm_solve* s, int32_t n) {
     HIPCHK(hipGraphLaunch(s->graph[s->parity], s->stream));
     // kGraphChunk is even, so the parity after the chunk is unchanged
     s->step += kGraphChunk;
-    s->force_pending = s->body && s->nslots;
     left -= kGraphChunk;
   }
   while (left-- > 0) {
@@ -1099,6 +1235,7 @@ int lbm_set_tile(lbm_solve* s, int32_t block_x, int32_t block_y, int32_t flags) 
   s->lin = (flags >> 2) & 1;
   s->occ = occ;
   s->tuned = true;
+  s->pair_rows = 0;  // the caller asks for this tile's launches
   int rc = build_force_slots(s);
   if (rc) return rc;
   return prepare_graphs(s);

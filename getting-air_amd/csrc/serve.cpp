@@ -512,7 +512,7 @@ int complete_chunk(lbm_serve* sv) {
       sv->finishing.push_back(std::move(m));
     } else {
       solve_advance(m->s, adv, false);
-      m->pending = m->entry.args[0].force_slot != nullptr;
+      m->pending = m->entry.args[0].boundary != nullptr;
       keep.push_back(std::move(m));
     }
   }
@@ -556,7 +556,7 @@ void retire(lbm_serve* sv) {
         rc = lbm_save_state(m.s, r.state_out.data(), n);
       }
     }
-    if (!rc && m.entry.args[0].force_slot) {
+    if (!rc && m.entry.args[0].boundary) {
       const int maxr = std::min(r.steps, 1 << 16);
       r.forces.resize((size_t)maxr * 6);
       int32_t cnt = 0;
