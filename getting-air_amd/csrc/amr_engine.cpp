@@ -733,7 +733,8 @@ int macro_step(lbm_amr* a) {
     HIPCHK(launch_pool_force(d.q, deep ? a->deep.back().pool[0] : a->pool[0], G,
                              deep ? a->deep.back().active : a->active, n, a->force_partials, a->stream));
     ForceSum fa{};
-    fa.partials[0] = a->force_partials;
+    fa.partials = a->force_partials;
+    fa.steps = 1;
     fa.nslots = pool_force_blocks(d.rb, n);
     fa.history = a->history;
     fa.written = a->written;

@@ -50,12 +50,15 @@ __host__ __device__ inline size_t lat_elem(int q, int i, uint32_t c) {
   return ((size_t)(c / kLatBlock) * q + i) * kLatBlock + c % kLatBlock;
 }
 
+// Steps a launch takes at most.
+constexpr int kMaxLaunchSteps = 8;
 // Force partials of a launch and where their sums go: slots summed in slot
 // order, one record [fx, fy, fz, tx, ty, tz] per step appended to the history
 // ring.
 struct ForceSum {
-  const double* partials[2];    // the launch's first step and, if it took two, its second (else null):
-                                // per slot [3] (force) with `cells`, else [6] (force and torque)
+  const double* partials;       // per slot [3] (force) with `cells`, else [6] (force and torque)
+  size_t stride;                // doubles from one step's slots to the next step's
+  int32_t steps;                // steps of the launch, kMaxLaunchSteps at most
   uint32_t nslots;
   const uint32_t* cells;        // per slot its boundary cell, or null
   double centre[3];             // torque arm origin
@@ -248,6 +251,23 @@ struct PairArgs {
 PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary);
 hipError_t launch_step_pair(int q, bool general, const void* fin, void* fout, const StepArgs& a, const PairArgs& p,
                             hipStream_t s);
+// Several D2Q9 steps in one launch (dense_multi.hip), on the bounce-back
+// coupling: gout holds the state `steps` steps after gin.
+constexpr int kMultiSmall = 1, kMultiDeep = 2, kMultiWide = 3;
+struct MultiPlan {
+  int32_t shape = 0;   // tile shape (kMulti*; 0: one-step launches)
+  int32_t steps = 0;   // steps a launch takes at most
+};
+struct MultiArgs {
+  int32_t steps;          // of this launch
+  int32_t ntx;
+  uint32_t nblocks;
+  size_t force_stride;    // doubles from one step's force slots to the next step's
+  int32_t finalize_prev;  // block 0 appends the previous launch's records (StepArgs::prev)
+};
+MultiPlan multi_plan(int q, int nx, int ny);
+hipError_t launch_step_multi(int storage, int shape, bool general, const void* fin, void* fout, const StepArgs& a,
+                             const MultiArgs& p, hipStream_t s);
 hipError_t launch_force_finalize(const ForceSum& a, hipStream_t s);
 hipError_t launch_totals(int q, int storage, const void* f, const TotalsArgs& a, int nblocks, hipStream_t s);
 // The wire format is plane-major f ([Q][ncells] float); the lattice uses the

@@ -24,7 +24,7 @@ namespace lbm {
 // cost the step kernels this is part of their occupancy).
 template <bool PERIODIC>
 __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, int part, int lane, double* out) {
-  const double* p = f.partials[rec];
+  const double* p = f.partials + (size_t)rec * f.stride;
   double v[6] = {0, 0, 0, 0, 0, 0};
   if (f.cells) {
     constexpr int B = PERIODIC ? 1 : 2;
@@ -70,12 +70,13 @@ __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, int p
     if (lane == 0) out[k] = t;
   }
 }
-// Appends the launch's records to the history; the whole block takes part.
-template <bool PERIODIC>
+// Appends the records of a launch of up to MAX steps to the history; the whole
+// block (64 threads or more) takes part.
+template <bool PERIODIC, int MAX>
 __device__ __forceinline__ void append_force_records(const ForceSum& f) {
-  __shared__ double part[2][4][6];
+  __shared__ double part[MAX][4][6];
   const int tid = threadIdx.x + threadIdx.y * blockDim.x, waves = (blockDim.x * blockDim.y) >> 6;
-  const int n = f.partials[1] ? 2 : 1;
+  const int n = MAX == 1 ? 1 : f.steps;
   for (int w = tid >> 6; w < 4 * n; w += waves)
     sum_force_wave<PERIODIC>(f, w >> 2, w & 3, tid & 63, part[w >> 2][w & 3]);
   __syncthreads();
@@ -121,6 +122,17 @@ __device__ __forceinline__ float body_phi(int shape, float radius, float cx, flo
 __device__ __forceinline__ bool on_wall_face(const StepArgs& a, int x, int y, int z) {
   return (a.wall_mask & 1 && (x == 0 || x == a.nx - 1)) || (a.wall_mask & 2 && (y == 0 || y == a.ny - 1)) ||
          (a.wall_mask & 4 && (z == 0 || z == a.nz - 1));
+}
+
+// Bit i set for the directions whose component on `axis` is v.
+template <int Q>
+__host__ __device__ constexpr uint32_t dirs_with(int axis, int v) {
+  uint32_t m = 0;
+  for (int i = 0; i < Q; i++) {
+    const int e = axis == 0 ? Lattice<Q>::ex[i] : (axis == 1 ? Lattice<Q>::ey[i] : Lattice<Q>::ez[i]);
+    if (e == v) m |= 1u << i;
+  }
+  return m;
 }
 
 // Halfway bounce-back of a cell next to the body (link mask `lm`) or on a

@@ -62,16 +62,6 @@ template <int Q>
 constexpr int lds_slots() {
   return Q - 3;  // all but (0, 0, -1), (0, 0, 0), (0, 0, 1)
 }
-// Bit i set for the directions whose component on `axis` is v.
-template <int Q>
-__host__ __device__ constexpr uint32_t dirs_with(int axis, int v) {
-  uint32_t m = 0;
-  for (int i = 0; i < Q; i++) {
-    const int e = axis == 0 ? Lattice<Q>::ex[i] : (axis == 1 ? Lattice<Q>::ey[i] : Lattice<Q>::ez[i]);
-    if (e == v) m |= 1u << i;
-  }
-  return m;
-}
 // Most rows of a block's column: 16 waves with the frame's, and two LDS buffers
 // of lds_slots directions of rows + 2 rows within the CU's 160 KiB.
 template <int Q>
@@ -109,7 +99,7 @@ k_step_pair(const float* __restrict__ gin, float* __restrict__ gout, StepArgs a,
     // also steps cells it would hold up all of that block's waves
     if (p.finalize_prev) {
       if (b == 0) {
-        append_force_records<false>(a.prev);
+        append_force_records<false, 2>(a.prev);
         return;
       }
       b--;

@@ -118,6 +118,21 @@ __device__ __forceinline__ void st_sr(typename ST::T* p, uint32_t i, float g, ui
   else *at(p, i) = v;
 }
 
+// Two stochastically rounded values of one cell, as stored.
+template <class ST>
+__device__ __forceinline__ void round_sr_pair(float gi, float gj, uint32_t ri, uint32_t rj, typename ST::T& hi,
+                                              typename ST::T& hj) {
+  if constexpr (std::is_same_v<ST, StoreF16>) {
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(__uint_as_float(__float_as_uint(gi) + ri),
+                                                                               __uint_as_float(__float_as_uint(gj) + rj)));
+    hi = (uint16_t)h;
+    hj = (uint16_t)(h >> 16);
+  } else {
+    hi = ST::round_sr(gi, ri);
+    hj = ST::round_sr(gj, rj);
+  }
+}
+
 // Two stochastically rounded stores of one cell (planes pi and pj).  binary16
 // converts both values with one packed round-toward-zero conversion, the
 // same bits as two single conversions.  The high half is taken from the

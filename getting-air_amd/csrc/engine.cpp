@@ -78,7 +78,8 @@ std::mutex g_tune_mu;
 std::map<TuneKey, TuneVal> g_tune_cache;
 
 const uint32_t kHistoryCap = 1u << 16;
-const int kGraphChunk = 16;  // steps per captured graph (even: parity returns)
+// launches per captured graph, of one step and of several (even: parity returns)
+const int kGraphChunk = 16, kGraphChunkMulti = 8;
 
 const int kEx9[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1}, kEy9[9] = {0, 0, 1, 0, -1, 1, 1, -1, -1};
 const int kEx3[27] = {0, 1, -1, 0, 0, 0, 0, 1, -1, 1, -1, 1, -1, 1, -1, 0, 0, 0, 0, 1, -1, 1, -1, 1, -1, 1, -1};
@@ -130,12 +131,14 @@ struct lbm_solve {
   int pair_rows = 0;                // two-step launches: rows of a block (0: none),
   PairBlock* pair_blocks = nullptr; // and the blocks
   uint32_t pair_nblocks = 0;
+  MultiPlan multi;                  // 2D launches of several steps (shape 0: none)
+  int force_subs = 1;               // steps of a launch the force partials hold
   bool tuned = false;
   bool initialised = false;
   long long step = 0;
   size_t bytes = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
-  int graph_bx = 0, graph_by = 0, graph_swz = 0, graph_nt = 0, graph_occ = 0, graph_lin = 0, graph_pair = 0;
+  int graph_bx = 0, graph_by = 0, graph_swz = 0, graph_nt = 0, graph_occ = 0, graph_lin = 0, graph_per = 0;
   Arena* arena = nullptr;           // pool the buffers come from (serve loop), or null
   bool own_stream = true;
   // Both parity graphs and the autotuned tile are made when the state is set
@@ -231,17 +234,18 @@ void pair_constants(StepArgs& a, const lbm_desc& d) {
 // CHI_EPS of the diffuse coupling (main-3d.js:1026 default 1.5).
 float chi_eps(const lbm_desc& d) { return d.chi_eps > 0.f ? d.chi_eps : 1.5f; }
 
-// Force slots of step `sub` (0, or 1: the second step of a two-step launch)
-// of a launch that read lattice `parity`.
+// Force slots: doubles of one step, steps of a launch, and the slots of step
+// `sub` of a launch that read lattice `parity`.
+size_t force_stride(const lbm_solve* s) { return (size_t)s->nslots * (s->d.diffuse ? 6 : 3); }
 double* force_set(const lbm_solve* s, int parity, int sub) {
-  const size_t width = s->d.diffuse ? 6 : 3, subs = s->arena ? 1 : 2;
-  return s->force_partials + (size_t)s->nslots * width * (parity * subs + sub);
+  return s->force_partials + force_stride(s) * (parity * s->force_subs + sub);
 }
 // The sum of the forces of a launch of `steps` steps that read lattice `parity`.
 ForceSum force_sum(const lbm_solve* s, int parity, int steps) {
   ForceSum f{};
-  f.partials[0] = force_set(s, parity, 0);
-  f.partials[1] = steps > 1 ? force_set(s, parity, 1) : nullptr;
+  f.partials = force_set(s, parity, 0);
+  f.stride = force_stride(s);
+  f.steps = steps;
   f.nslots = s->nslots;
   f.cells = s->d.diffuse ? nullptr : s->boundary_cells;
   f.centre[0] = s->d.body.centre[0];
@@ -330,8 +334,8 @@ int build_boundary_slots(lbm_solve* s) {
   }
   s->rank_bytes = groups * sizeof(BoundaryRank);
   s->cell_bytes = std::max<size_t>(n, 1) * 4;
-  // one set per lattice parity and step of a launch (one step in a pool)
-  s->partial_bytes = (size_t)(s->arena ? 2 : 4) * std::max<size_t>(n, 1) * 3 * 8;
+  // one set per lattice parity and step of a launch
+  s->partial_bytes = (size_t)2 * s->force_subs * std::max<size_t>(n, 1) * 3 * 8;
   int rc = dalloc(s, &s->ranks, s->rank_bytes);
   if (!rc) rc = dalloc(s, &s->boundary_cells, s->cell_bytes);
   if (!rc) rc = dalloc(s, &s->force_partials, s->partial_bytes);
@@ -380,7 +384,7 @@ int build_force_slots(lbm_solve* s) {
   s->force_slot = nullptr;
   s->force_partials = nullptr;
   s->slot_bytes = ntiles * 4;
-  s->partial_bytes = 2 * 2 * std::max<size_t>(n, 1) * 6 * 8;  // as force_set lays them out
+  s->partial_bytes = 2 * std::max<size_t>(n, 1) * 6 * 8;  // one set per lattice parity
   int rc = dalloc(s, &s->force_slot, s->slot_bytes);
   if (rc) return rc;
   rc = dalloc(s, &s->force_partials, s->partial_bytes);
@@ -438,8 +442,34 @@ int enqueue_pair(lbm_solve* s, bool write_mac, bool finalize_prev) {
   return LBM_OK;
 }
 
-// Whether this solve's steps may go in pairs now.
-bool pairs_on(const lbm_solve* s) { return s->pair_rows > 0 && !s->rigid; }
+// `steps` 2D steps in one launch.
+int enqueue_multi(lbm_solve* s, int steps, bool write_mac, bool finalize_prev) {
+  StepArgs a = step_args(s, write_mac, true);
+  a.finalize_prev = finalize_prev && a.boundary ? 1 : 0;
+  a.prev = a.boundary ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
+  MultiArgs p{};
+  p.steps = steps;
+  p.force_stride = force_stride(s);
+  hipError_t e = launch_step_multi(s->storage, s->multi.shape, s->general, s->f[s->parity], s->f[1 - s->parity], a, p,
+                                   s->stream);
+  if (e != hipSuccess) return hip_fail(e, "multi-step kernel launch");
+  s->force_pending = a.boundary ? steps : 0;
+  s->parity ^= 1;
+  s->step += steps;
+  return LBM_OK;
+}
+
+// Steps a launch of this solve takes now.
+int launch_steps(const lbm_solve* s) {
+  if (s->pair_rows > 0 && !s->rigid) return 2;
+  return s->multi.shape && !s->rigid ? s->multi.steps : 1;
+}
+
+// A launch of `steps` steps, launch_steps or (2D, or a single step) fewer.
+int enqueue_launch(lbm_solve* s, int steps, bool write_mac, bool finalize_prev) {
+  if (s->multi.shape) return enqueue_multi(s, steps, write_mac, finalize_prev);
+  return steps == 2 ? enqueue_pair(s, write_mac, finalize_prev) : enqueue_step(s, write_mac, finalize_prev);
+}
 
 // Appends the force records of the last enqueued launch.
 int flush_force(lbm_solve* s) {
@@ -487,23 +517,20 @@ void drop_graphs(lbm_solve* s) {
   }
 }
 
-// Captures kGraphChunk steps starting at the current parity (an even number of
-// launches, also in pairs, so the parity returns).
+int chunk_launches(const lbm_solve* s) { return launch_steps(s) > 1 ? kGraphChunkMulti : kGraphChunk; }
+
+// Captures a chunk of launches starting at the current parity.
 int build_graph(lbm_solve* s) {
   const int p = s->parity;
   hipGraph_t g = nullptr;
   HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
   const long long step0 = s->step;
   const int pending0 = s->force_pending;
-  const bool pairs = pairs_on(s);
+  const int per = launch_steps(s);
   // a chunk follows a launch of its own kind (lbm_step)
-  s->force_pending = s->body && s->nslots ? (pairs ? 2 : 1) : 0;
+  s->force_pending = s->body && s->nslots ? per : 0;
   int rc = LBM_OK;
-  if (pairs) {
-    for (int k = 0; k < kGraphChunk / 2 && rc == LBM_OK; k++) rc = enqueue_pair(s, false, true);
-  } else {
-    for (int k = 0; k < kGraphChunk && rc == LBM_OK; k++) rc = enqueue_step(s, false, true);
-  }
+  for (int k = 0; k < chunk_launches(s) && rc == LBM_OK; k++) rc = enqueue_launch(s, per, false, true);
   hipError_t e = hipStreamEndCapture(s->stream, &g);
   s->step = step0;
   s->parity = p;
@@ -518,14 +545,14 @@ int build_graph(lbm_solve* s) {
   if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
   s->graph_bx = s->bx; s->graph_by = s->by; s->graph_swz = s->swz; s->graph_nt = s->nt; s->graph_occ = s->occ;
   s->graph_lin = s->lin;
-  s->graph_pair = pairs;
+  s->graph_per = per;
   return LBM_OK;
 }
 
 // Whether the captured chunks are of the current tile and launch form.
 bool graphs_current(const lbm_solve* s) {
   return s->graph_bx == s->bx && s->graph_by == s->by && s->graph_swz == s->swz && s->graph_nt == s->nt &&
-         s->graph_occ == s->occ && s->graph_lin == s->lin && s->graph_pair == (int)pairs_on(s);
+         s->graph_occ == s->occ && s->graph_lin == s->lin && s->graph_per == launch_steps(s);
 }
 
 int autotune(lbm_solve* s);
@@ -724,6 +751,11 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
     s->nt = (flags >> 1) & 1;
     s->lin = (flags >> 2) & 1;
     s->occ = (flags >> 4) & 15;
+  }
+  // launches of several steps (a pool member's steps are the batched kernel's)
+  if (!arena && !desc->diffuse) {
+    s->multi = multi_plan(s->q, desc->nx, desc->ny);
+    s->force_subs = s->dim == 2 ? std::max(1, s->multi.steps) : 2;
   }
   hipError_t e = hipSuccess;
   if (stream) {
@@ -1060,22 +1092,24 @@ int lbm_step(lbm_solve* s, int32_t n) {
   }
   if (!graphs_current(s)) drop_graphs(s);
   int rc = LBM_OK;
-  if (pairs_on(s)) {
-    // An odd step first, then pairs: one eagerly (so that every chunk follows
-    // a pair, whose forces its first launch sums), captured chunks, single
-    // pairs, the last of them writing the macroscopic field.
-    if (n & 1) rc = enqueue_step(s, n == 1, false);
-    int left = n / 2;
+  const int per = launch_steps(s);
+  if (per > 1) {
+    // The steps that do not fill a launch first, then whole launches: one
+    // eagerly (so that every chunk follows a launch of its own kind, whose
+    // forces its first launch sums), captured chunks, single launches, the
+    // last of them writing the macroscopic field.
+    if (n % per) rc = enqueue_launch(s, n % per, n < per, false);
+    int left = n / per;
     bool first = true;
     while (left > 0 && rc == LBM_OK) {
-      if (!first && left > kGraphChunk / 2) {
+      if (!first && left > chunk_launches(s)) {
         if (!s->graph[s->parity] && (rc = build_graph(s))) return rc;
         HIPCHK(hipGraphLaunch(s->graph[s->parity], s->stream));
-        s->step += kGraphChunk;
-        left -= kGraphChunk / 2;
+        s->step += chunk_launches(s) * per;
+        left -= chunk_launches(s);
         continue;
       }
-      rc = enqueue_pair(s, left == 1, s->force_pending != 0);
+      rc = enqueue_launch(s, per, left == 1, s->force_pending != 0);
       first = false;
       left--;
     }
@@ -1236,6 +1270,7 @@ int lbm_set_tile(lbm_solve* s, int32_t block_x, int32_t block_y, int32_t flags) 
   s->occ = occ;
   s->tuned = true;
   s->pair_rows = 0;  // the caller asks for this tile's launches
+  s->multi = MultiPlan{};
   int rc = build_force_slots(s);
   if (rc) return rc;
   return prepare_graphs(s);
