@@ -15,6 +15,7 @@
 #include "amr.h"
 #include "engine.h"
 #include "lattice_pairs.h"
+#include "readback.h"
 
 using namespace lbm;
 
@@ -1220,13 +1221,7 @@ int lbm_amr_read_forces(lbm_amr* a, double* out, int32_t max_records, int32_t* c
   HIPCHK(hipStreamSynchronize(a->stream));
   const unsigned long long avail = std::min<unsigned long long>(written, kForceCap);
   const unsigned long long take = std::min<unsigned long long>(avail, (unsigned long long)std::max(0, max_records));
-  if (take) {
-    std::vector<double> ring((size_t)kForceCap * 6);
-    HIPCHK(hipMemcpyAsync(ring.data(), a->history, ring.size() * 8, hipMemcpyDeviceToHost, a->stream));
-    HIPCHK(hipStreamSynchronize(a->stream));
-    for (unsigned long long k = 0; k < take; k++)
-      memcpy(out + k * 6, ring.data() + ((written - take + k) % kForceCap) * 6, 48);
-  }
+  HIPCHK(read_records(out, a->history, kForceCap, written, take, a->stream));
   *count = (int32_t)take;
   return LBM_OK;
 }

@@ -24,6 +24,7 @@
 
 #include "../../include/lbm.h"
 #include "dense.h"
+#include "readback.h"
 #include "rigid.h"
 #include "engine.h"
 #include "lattice_pairs.h"
@@ -711,6 +712,7 @@ void release(lbm_solve* s) {
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   if (s->stream && s->own_stream) (void)hipStreamDestroy(s->stream);
+  read_back_release();
   delete s;
 }
 
@@ -733,6 +735,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
   int rc = validate(desc);
   if (rc) return rc;
   lbm_solve* s = new lbm_solve();
+  read_back_retain();
   s->arena = arena;
   s->eager_graphs = arena == nullptr;
   s->d = *desc;
@@ -1168,8 +1171,7 @@ int lbm_sync(lbm_solve* s) {
 
 int lbm_read_macro(lbm_solve* s, float* mac4) {
   if (!s || !mac4) return fail(LBM_E_INVALID, "null argument");
-  HIPCHK(hipMemcpyAsync(mac4, s->mac, (size_t)s->N * 16, hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
+  HIPCHK(read_back(mac4, s->mac, (size_t)s->N * 16, s->stream));
   return LBM_OK;
 }
 
@@ -1180,16 +1182,7 @@ int lbm_read_forces(lbm_solve* s, double* out, int32_t max_records, int32_t* cou
   HIPCHK(hipStreamSynchronize(s->stream));
   const unsigned long long avail = std::min<unsigned long long>(written, kHistoryCap);
   const unsigned long long take = std::min<unsigned long long>(avail, (unsigned long long)std::max(0, max_records));
-  // the `take` most recent records, oldest first
-  if (take) {
-    std::vector<double> ring((size_t)kHistoryCap * 6);
-    HIPCHK(hipMemcpyAsync(ring.data(), s->history, ring.size() * 8, hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
-    for (unsigned long long k = 0; k < take; k++) {
-      const unsigned long long rec = written - take + k;
-      memcpy(out + k * 6, ring.data() + (rec % kHistoryCap) * 6, 48);
-    }
-  }
+  HIPCHK(read_records(out, s->history, kHistoryCap, written, take, s->stream));
   *count = (int32_t)take;
   return LBM_OK;
 }
