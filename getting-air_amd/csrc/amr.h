@@ -149,11 +149,17 @@ hipError_t launch_cell_class(int q, uint8_t* ccls, const PoolGeom& g, const Surf
 hipError_t launch_pool_step(int q, const float* gin, float* gout, float* mac_pool, const PoolGeom& g,
                             const CollideParams& fine, int nactive, int collide_ring, int sub, hipStream_t s);
 // Momentum exchange on the fine-level body from the pool state at the start
-// of the macro-step: one FP64 [fx, fy, fz, tx, ty, tz] partial per thread
-// block (pool_force_blocks of them), weighted dx^2 = 1/4.
+// of the macro-step (gp), taken by explode's launch: one FP64 [fx, fy, fz, tx,
+// ty, tz] partial per thread block (pool_force_blocks of them), weighted dx^2 =
+// 1/4, which coalesce's launch sums into the record.
 uint32_t pool_force_blocks(int rb, int nactive);
-hipError_t launch_pool_force(int q, const float* gpool, const PoolGeom& g, const int32_t* active, int nactive,
-                             double* partials, hipStream_t s);
+struct PoolForce {
+  const float* gp;
+  PoolGeom G;
+  const int32_t* active;
+  int32_t nactive;
+  double* partials;
+};
 // Seam flux of the fine solver over one substep, from the pool buffer that
 // substep streams: [dm, dpx, dpy, dpz] / 8 per flux cell, written
 // (accumulate 0) or added (1).
@@ -164,11 +170,13 @@ hipError_t launch_flux(int q, const float* gpool, float* acc, const PoolGeom& g,
 hipError_t launch_reflux(int q, const float* gc_t, float* gc_t1, float* mac, const PoolGeom& g, const SurfacePlan& plan,
                          uint32_t nflux, float* acc, const float* force, hipStream_t s);
 // dirs: directions per thread (0: about 2^20 threads for the ring).
+// force: the body's force pass, or null (dense parent only).
 hipError_t launch_explode(int q, const ParentRef& parent, float* gpool, const PoolGeom& g, const SurfacePlan& plan,
-                          uint32_t nring, int linear, int dirs, hipStream_t s);
+                          uint32_t nring, int linear, int dirs, const PoolForce* force, hipStream_t s);
+// force: the record of the macro-step's force pass, or null (dense parent only).
 hipError_t launch_coalesce(int q, const float* gpool, const ParentRef& parent, const float* mac_pool,
                            const PoolGeom& g, const int32_t* active, int nactive, const SurfacePlan& plan,
-                           uint32_t nseam, uint32_t nnear, int orphans, hipStream_t s);
+                           uint32_t nseam, uint32_t nnear, int orphans, const ForceSum* force, hipStream_t s);
 // ring_only: the ring cells alone (the interp interface's per-step refresh).
 // A pool parent is sampled in the parent tile that holds the child block
 // (its ring included), at the parent's own time level.

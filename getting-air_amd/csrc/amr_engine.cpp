@@ -692,13 +692,14 @@ int advance(lbm_amr* a, int m, int p) {
     DeepLevel& c = a->deep[m - 1];
     if (c.nactive > 0) {
       const ParentRef P = pool_parent(a, m, p);
-      HIPCHK(launch_explode(d.q, P, c.pool[0], c.G, c.plan, c.nring, d.explode_linear, d.explode_dirs, a->stream));
+      HIPCHK(launch_explode(d.q, P, c.pool[0], c.G, c.plan, c.nring, d.explode_linear, d.explode_dirs, nullptr,
+                            a->stream));
       int rc = advance(a, m + 1, 0);
       if (rc) return rc;
       rc = advance(a, m + 1, 1);
       if (rc) return rc;
       HIPCHK(launch_coalesce(d.q, c.pool[0], P, c.mac_pool, c.G, c.active, c.nactive, c.plan, c.nseam, c.nnear,
-                             d.orphans, a->stream));
+                             d.orphans, nullptr, a->stream));
     }
   }
   if (m == 1) {
@@ -725,31 +726,33 @@ int macro_step(lbm_amr* a) {
     return LBM_OK;
   }
   float* l0 = solve_lattice(a->l0, 0);
+  PoolForce force{};
+  ForceSum record{};
   if (a->has_body) {
     // the one force pass of the macro-step, on the finest level's state at t
     // (main-3d.js:3127-3141, 1596-1597)
     const bool deep = a->levels > 2;
-    const PoolGeom& G = deep ? a->deep.back().G : a->G;
-    const int n = deep ? a->deep.back().nactive : a->nactive;
-    HIPCHK(launch_pool_force(d.q, deep ? a->deep.back().pool[0] : a->pool[0], G,
-                             deep ? a->deep.back().active : a->active, n, a->force_partials, a->stream));
-    ForceSum fa{};
-    fa.partials = a->force_partials;
-    fa.steps = 1;
-    fa.nslots = pool_force_blocks(d.rb, n);
-    fa.history = a->history;
-    fa.written = a->written;
-    fa.capacity = kForceCap;
-    HIPCHK(launch_force_finalize(fa, a->stream));
+    force.gp = deep ? a->deep.back().pool[0] : a->pool[0];
+    force.G = deep ? a->deep.back().G : a->G;
+    force.active = deep ? a->deep.back().active : a->active;
+    force.nactive = deep ? a->deep.back().nactive : a->nactive;
+    force.partials = a->force_partials;
+    record.partials = a->force_partials;
+    record.steps = 1;
+    record.nslots = pool_force_blocks(d.rb, force.nactive);
+    record.history = a->history;
+    record.written = a->written;
+    record.capacity = kForceCap;
   }
   const ParentRef P0 = dense_parent(a, l0);
-  HIPCHK(launch_explode(d.q, P0, a->pool[0], a->G, a->plan, a->nring, d.explode_linear, d.explode_dirs, a->stream));
+  HIPCHK(launch_explode(d.q, P0, a->pool[0], a->G, a->plan, a->nring, d.explode_linear, d.explode_dirs,
+                        a->has_body ? &force : nullptr, a->stream));
   int rc0 = advance(a, 1, 0);
   if (rc0) return rc0;
   rc0 = advance(a, 1, 1);
   if (rc0) return rc0;
   HIPCHK(launch_coalesce(d.q, a->pool[0], P0, a->mac_pool, a->G, a->active, a->nactive, a->plan, a->nseam, a->nnear,
-                         d.orphans, a->stream));
+                         d.orphans, a->has_body ? &record : nullptr, a->stream));
   int rc = solve_enqueue_covered_step(a->l0, a->block_slot, d.rb, a->G.nbx, a->G.nby);
   if (rc) return rc;
   a->step++;

@@ -33,6 +33,8 @@
 
 #include "amr.h"
 #include "collide.h"
+#include "dense.h"
+#include "dense_cell.h"
 #include "device_common.h"
 #include "lattice_pairs.h"
 #include "lattice_tables.h"
@@ -99,10 +101,11 @@ using TileQ = Tile<RB, Lattice<Q>::D>;
 // keeps a tile's blocks, and the neighbouring rows and planes their pulls
 // share, in one L2 (without it the pool step fetched 2.5x its algorithmic
 // bytes from HBM).
-__device__ __forceinline__ uint32_t xcd_block() {
-  const uint32_t b = blockIdx.x, per = gridDim.x >> 3;
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t n) {
+  const uint32_t per = n >> 3;
   return b < per * 8u ? (b & 7u) * per + (b >> 3) : b;
 }
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 // Tile index of a tile-major launch, made wave-uniform (scalar registers)
 // where a wave lies in one tile (3D); per lane for a 2D tile, which is not a
@@ -535,16 +538,17 @@ k_pool_step(const float* __restrict__ gin, float* __restrict__ gout, float* __re
 // units.  One thread per interior cell of each active tile; each block leaves
 // its FP64 partial in `partials`, summed in block order afterwards.
 template <int Q, int RB>
-__global__ void __launch_bounds__(256)
-k_pool_force(const float* __restrict__ gp, PoolGeom G, const int32_t* __restrict__ active, int nactive,
-             double* __restrict__ partials) {
+__device__ __forceinline__ void pool_force_block(const PoolForce& f, uint32_t block) {
   using L = Lattice<Q>;
   constexpr int RB2 = 2 * RB;
   constexpr uint32_t per = RB2 * RB2 * RB2;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const PoolGeom& G = f.G;
+  const float* const gp = f.gp;
+  const int32_t* const active = f.active;
+  const uint32_t t = block * blockDim.x + threadIdx.x;
   const uint32_t k = t / per;
   double fv[6] = {0, 0, 0, 0, 0, 0};
-  if (k < (uint32_t)nactive) {
+  if (k < (uint32_t)f.nactive) {
     const uint32_t r = t - k * per;
     const int fx = kGhost + (int)(r % RB2), fy = kGhost + (int)((r / RB2) % RB2), fz = kGhost + (int)(r / (RB2 * RB2));
     const int slot = active[1 + k];
@@ -583,40 +587,40 @@ k_pool_force(const float* __restrict__ gp, PoolGeom G, const int32_t* __restrict
   block_sum<6>(fv, lds);
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int c = 0; c < 6; c++) partials[(size_t)blockIdx.x * 6 + c] = fv[c];
+    for (int c = 0; c < 6; c++) f.partials[(size_t)block * 6 + c] = fv[c];
   }
 }
 
 // ---------------------------------------------------------------------------
 // explode: coarse state at t -> ring of the pool buffer the first substep reads
 // ---------------------------------------------------------------------------
-// Bit i set for the directions whose component on `axis` is v.
-template <int Q>
-__device__ constexpr uint32_t dirs_with(int axis, int v) {
-  uint32_t m = 0;
-  for (int i = 0; i < Q; i++) {
-    const int e = axis == 0 ? Lattice<Q>::ex[i] : (axis == 1 ? Lattice<Q>::ey[i] : Lattice<Q>::ez[i]);
-    if (e == v) m |= 1u << i;
-  }
-  return m;
-}
-template <int Q, int RB, bool PP>
+// FORCE: the blocks past explode's nblocks x groups take the body's force pass,
+// which reads interior cells of the state at t where explode writes ring cells.
+// Both are short of waves (AMR sphere, 192 x 128 x 128, rb 4: 8.5 and 11.3 us).
+template <int Q, int RB, bool PP, bool FORCE>
 __global__ void __launch_bounds__(256)
 k_explode(ParentRef P, float* __restrict__ gp, PoolGeom G, const uint4* __restrict__ ring, uint32_t nring, int linear,
-          int per) {
+          int per, uint32_t nblocks, uint32_t groups, PoolForce force) {
   using L = Lattice<Q>;
   using T = TileQ<Q, RB>;
   constexpr int LO = T::LO, HI = T::HI;
-  const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
+  if constexpr (FORCE) {
+    if (blockIdx.x >= nblocks * groups) {
+      pool_force_block<Q, RB>(force, blockIdx.x - nblocks * groups);
+      return;
+    }
+  }
+  const uint32_t group = blockIdx.x / nblocks;
+  const uint32_t t = xcd_block(blockIdx.x - group * nblocks, nblocks) * blockDim.x + threadIdx.x;
   if (t >= nring) return;
   const uint4 d = ring[t];
   if (d.x == kAbsent) return;  // the L0 cell under this ring cell is refined
-  // Grid row g takes directions [g per, (g + 1) per): a ring cell's Q
+  // Group g takes directions [g per, (g + 1) per): a ring cell's Q
   // populations are independent, so a small ring spreads them over threads
   // (one thread per ring cell leaves too few waves to hide the loads) and a
   // large one keeps them in one thread (which shares the index work among
   // them).
-  const int i0 = (int)blockIdx.y * per, i1 = min(Q, i0 + per);
+  const int i0 = (int)group * per, i1 = min(Q, i0 + per);
   // a ring cell over an unrefined L0 cell, and its explode decisions
   // (k_ring_plan)
   const uint32_t cell = d.x, vc = d.y, bits = d.z;
@@ -693,13 +697,12 @@ k_explode(ParentRef P, float* __restrict__ gp, PoolGeom G, const uint4* __restri
 // mac projection of every covered L0 cell from its 8 children (4 in 2D;
 // rho mean, mass-weighted u; common_d3_amr_coalesce.wgsl:245-261)
 template <int Q, int RB, bool PP>
-__global__ void __launch_bounds__(256)
-k_coalesce_mac(ParentRef P, const float* __restrict__ mac_pool, PoolGeom G, const int32_t* __restrict__ active,
-               int nactive) {
+__device__ __forceinline__ void coalesce_mac(const ParentRef& P, const float* __restrict__ mac_pool, const PoolGeom& G,
+                                             const int32_t* __restrict__ active, int nactive, uint32_t block) {
   using T = TileQ<Q, RB>;
   constexpr int D = Lattice<Q>::D;
   constexpr uint32_t per = D == 3 ? RB * RB * RB : RB * RB;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = block * blockDim.x + threadIdx.x;
   const uint32_t k = t / per;
   if (k >= (uint32_t)nactive) return;
   const uint32_t r = t - k * per;
@@ -726,16 +729,14 @@ k_coalesce_mac(ParentRef P, const float* __restrict__ mac_pool, PoolGeom G, cons
 
 // Covered seam cells: for every direction whose target is unrefined, the
 // mean of the 8 ring cells covering the target (common_d3_amr_coalesce.wgsl:
-// 264-284).  One thread per (seam cell, direction i = 1 + grid row).
+// 264-284).  One thread per (seam cell, direction i).
 template <int Q, int RB, bool PP>
-__global__ void __launch_bounds__(256)
-k_coalesce_seam(const float* __restrict__ gp, ParentRef P, PoolGeom G, const uint32_t* __restrict__ seam,
-                uint32_t nseam) {
+__device__ __forceinline__ void coalesce_seam(const float* __restrict__ gp, const ParentRef& P, const PoolGeom& G,
+                                              const uint32_t* __restrict__ seam, uint32_t nseam, uint32_t block, int i) {
   using T = TileQ<Q, RB>;
   constexpr int FB = T::FB, D = Lattice<Q>::D;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = block * blockDim.x + threadIdx.x;
   if (t >= nseam) return;
-  const int i = 1 + blockIdx.y;
   int ex, ey, ez;
   float wi;
   direction<Q>(i, ex, ey, ez, wi);
@@ -761,16 +762,16 @@ k_coalesce_seam(const float* __restrict__ gp, ParentRef P, PoolGeom G, const uin
 
 // Orphans on unrefined L0 cells next to the refined region
 // (coalesceOrphans, common_d3_amr_coalesce.wgsl:126-211).  One thread per
-// (near cell, direction i = 1 + grid row); the 8 child lookups of a
-// direction are independent loads.
+// (near cell, direction i); the 8 child lookups of a direction are independent
+// loads.
 template <int Q, int RB, bool PP>
-__global__ void __launch_bounds__(256)
-k_orphans(const float* __restrict__ gp, ParentRef P, PoolGeom G, const uint32_t* __restrict__ near, uint32_t nnear) {
+__device__ __forceinline__ void coalesce_orphans(const float* __restrict__ gp, const ParentRef& P, const PoolGeom& G,
+                                                 const uint32_t* __restrict__ near, uint32_t nnear, uint32_t block,
+                                                 int i) {
   using T = TileQ<Q, RB>;
   constexpr int D = Lattice<Q>::D;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = block * blockDim.x + threadIdx.x;
   if (t >= nnear) return;
-  const int i = 1 + blockIdx.y;
   int ex, ey, ez;
   float wi;
   direction<Q>(i, ex, ey, ez, wi);
@@ -804,6 +805,37 @@ k_orphans(const float* __restrict__ gp, ParentRef P, PoolGeom G, const uint32_t*
   const float fc = gci + wi;
   const float net = s - nIn * fc;
   if (net != 0.f) gci = (fc + net * T::INV_NCH) - wi;
+}
+
+// The three passes in one launch: they write apart (macroscopic field and
+// populations of covered cells, populations of uncovered ones) and read nothing
+// that another writes.  Blocks in order: orphans, whose chains of dependent
+// loads are the longest, seam, macroscopic field, and, with a body, one that
+// appends the force record of the pass before (PoolForce).
+template <int Q, int RB, bool PP>
+__global__ void __launch_bounds__(256)
+k_coalesce(const float* __restrict__ gp, ParentRef P, const float* __restrict__ mac_pool, PoolGeom G,
+           const int32_t* __restrict__ active, int nactive, const uint32_t* __restrict__ seam, uint32_t nseam,
+           const uint32_t* __restrict__ near, uint32_t nnear, uint32_t seam_blocks, uint32_t near_blocks,
+           uint32_t mac_blocks, ForceSum force) {
+  uint32_t b = blockIdx.x;
+  if (b < near_blocks * (Q - 1)) {
+    const uint32_t row = b / near_blocks;
+    coalesce_orphans<Q, RB, PP>(gp, P, G, near, nnear, b - row * near_blocks, 1 + (int)row);
+    return;
+  }
+  b -= near_blocks * (Q - 1);
+  if (b < seam_blocks * (Q - 1)) {
+    const uint32_t row = b / seam_blocks;
+    coalesce_seam<Q, RB, PP>(gp, P, G, seam, nseam, b - row * seam_blocks, 1 + (int)row);
+    return;
+  }
+  b -= seam_blocks * (Q - 1);
+  if (b < mac_blocks) {
+    coalesce_mac<Q, RB, PP>(P, mac_pool, G, active, nactive, b);
+    return;
+  }
+  if constexpr (!PP && Lattice<Q>::D == 3) append_force_records<false, 1>(force);
 }
 
 // ---------------------------------------------------------------------------
@@ -1426,15 +1458,6 @@ struct OpPoolStep {
   }
 };
 template <int Q, int RB>
-struct OpPoolForce {
-  static hipError_t run(const float* gp, const PoolGeom& g, const int32_t* active, int nactive, double* partials,
-                        hipStream_t s) {
-    hipLaunchKernelGGL((k_pool_force<Q, RB>), dim3(pool_force_blocks(RB, nactive)), dim3(256), 0, s, gp, g, active,
-                       nactive, partials);
-    return hipGetLastError();
-  }
-};
-template <int Q, int RB>
 struct OpFlux {
   static hipError_t run(const float* gp, float* acc, const PoolGeom& g, const SurfacePlan& plan, uint32_t n,
                         int accumulate, hipStream_t s) {
@@ -1455,15 +1478,24 @@ struct OpReflux {
 template <int Q, int RB>
 struct OpExplode {
   static hipError_t run(const ParentRef& P, float* gp, const PoolGeom& g, const SurfacePlan& plan, uint32_t nring,
-                        int linear, int dirs, hipStream_t s) {
+                        int linear, int dirs, const PoolForce* force, hipStream_t s) {
     // about 2^20 threads: every direction its own thread for a small ring,
     // all Q in one thread for a ring of a million cells
-    const int groups = (int)std::min<uint64_t>(Q, std::max<uint64_t>(1, ((1u << 20) + nring - 1) / nring));
-    const int per = dirs > 0 ? std::min(dirs, Q) : (Q + groups - 1) / groups;
-    with_parent(P, [&](auto PP) {
-      hipLaunchKernelGGL((k_explode<Q, RB, decltype(PP)::value>), grid_for(nring, (Q + per - 1) / per), dim3(256), 0,
-                         s, P, gp, g, plan.ring, nring, linear, per);
-    });
+    const int split = (int)std::min<uint64_t>(Q, std::max<uint64_t>(1, ((1u << 20) + nring - 1) / nring));
+    const int per = dirs > 0 ? std::min(dirs, Q) : (Q + split - 1) / split;
+    const uint32_t nblocks = grid_for(nring).x, groups = (Q + per - 1) / per;
+    auto go = [&](auto PP, auto F, uint32_t extra) {
+      hipLaunchKernelGGL((k_explode<Q, RB, decltype(PP)::value, decltype(F)::value>), dim3(nblocks * groups + extra),
+                         dim3(256), 0, s, P, gp, g, plan.ring, nring, linear, per, nblocks, groups,
+                         force ? *force : PoolForce{});
+    };
+    if constexpr (Lattice<Q>::D == 3) {
+      if (force) {
+        go(std::false_type{}, std::true_type{}, pool_force_blocks(RB, force->nactive));
+        return hipGetLastError();
+      }
+    }
+    with_parent(P, [&](auto PP) { go(PP, std::false_type{}, 0); });
     return hipGetLastError();
   }
 };
@@ -1471,18 +1503,15 @@ template <int Q, int RB>
 struct OpCoalesce {
   static hipError_t run(const float* gp, const ParentRef& P, const float* mac_pool, const PoolGeom& g,
                         const int32_t* active, int nactive, const SurfacePlan& plan, uint32_t nseam, uint32_t nnear,
-                        int orphans, hipStream_t s) {
+                        int orphans, const ForceSum* force, hipStream_t s) {
+    const uint32_t mac_blocks = grid_for((uint64_t)nactive * parent_cells<Q, RB>()).x, seam_blocks = grid_for(nseam).x,
+                   near_blocks = orphans ? grid_for(nnear).x : 0;
+    const uint32_t blocks = mac_blocks + (seam_blocks + near_blocks) * (Q - 1) + (force ? 1 : 0);
+    if (blocks == 0) return hipSuccess;
     with_parent(P, [&](auto PP) {
-      constexpr bool pp = decltype(PP)::value;
-      if (nactive > 0)
-        hipLaunchKernelGGL((k_coalesce_mac<Q, RB, pp>), grid_for((uint64_t)nactive * parent_cells<Q, RB>()), dim3(256), 0, s, P,
-                           mac_pool, g, active, nactive);
-      if (nseam > 0)
-        hipLaunchKernelGGL((k_coalesce_seam<Q, RB, pp>), grid_for(nseam, Q - 1), dim3(256), 0, s, gp, P, g, plan.seam,
-                           nseam);
-      if (orphans && nnear > 0)
-        hipLaunchKernelGGL((k_orphans<Q, RB, pp>), grid_for(nnear, Q - 1), dim3(256), 0, s, gp, P, g, plan.near,
-                           nnear);
+      hipLaunchKernelGGL((k_coalesce<Q, RB, decltype(PP)::value>), dim3(blocks), dim3(256), 0, s, gp, P, mac_pool, g,
+                         active, nactive, plan.seam, nseam, plan.near, nnear, seam_blocks, near_blocks, mac_blocks,
+                         force ? *force : ForceSum{});
     });
     return hipGetLastError();
   }
@@ -1541,10 +1570,6 @@ uint32_t pool_force_blocks(int rb, int nactive) {
   const uint64_t per = (uint64_t)(2 * rb) * (2 * rb) * (2 * rb);
   return (uint32_t)std::max<uint64_t>(1, ((uint64_t)std::max(0, nactive) * per + 255) / 256);
 }
-hipError_t launch_pool_force(int q, const float* gpool, const PoolGeom& g, const int32_t* active, int nactive,
-                             double* partials, hipStream_t s) {
-  return dispatch_q3_rb<OpPoolForce>(q, g.rb, gpool, g, active, nactive, partials, s);
-}
 hipError_t launch_flux(int q, const float* gp, float* acc, const PoolGeom& g, const SurfacePlan& plan, uint32_t nflux,
                        int accumulate, hipStream_t s) {
   if (nflux == 0) return hipSuccess;
@@ -1557,16 +1582,18 @@ hipError_t launch_reflux(int q, const float* gct, float* gct1, float* mac, const
 }
 
 hipError_t launch_explode(int q, const ParentRef& parent, float* gp, const PoolGeom& g, const SurfacePlan& plan,
-                          uint32_t nring, int linear, int dirs, hipStream_t s) {
+                          uint32_t nring, int linear, int dirs, const PoolForce* force, hipStream_t s) {
+  // a body always lies in some tile
+  if (force && (nring == 0 || force->nactive <= 0)) return hipErrorInvalidConfiguration;
   if (nring == 0) return hipSuccess;
-  return dispatch_q_rb<OpExplode>(q, g.rb, parent, gp, g, plan, nring, linear, dirs, s);
+  return dispatch_q_rb<OpExplode>(q, g.rb, parent, gp, g, plan, nring, linear, dirs, force, s);
 }
 
 hipError_t launch_coalesce(int q, const float* gp, const ParentRef& parent, const float* mac_pool, const PoolGeom& g,
                            const int32_t* active, int nactive, const SurfacePlan& plan, uint32_t nseam,
-                           uint32_t nnear, int orphans, hipStream_t s) {
+                           uint32_t nnear, int orphans, const ForceSum* force, hipStream_t s) {
   return dispatch_q_rb<OpCoalesce>(q, g.rb, gp, parent, mac_pool, g, active, nactive, plan, nseam, nnear, orphans,
-                                   s);
+                                   force, s);
 }
 
 hipError_t launch_interp(int q, const ParentRef& parent, float* gp, const PoolGeom& g, const int32_t* pairs,
