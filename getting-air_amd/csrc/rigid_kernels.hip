@@ -98,8 +98,14 @@ __device__ void rigid_physics(RigidBody* B, const double F[3], const double T[3]
 
 }  // namespace
 
+// Cells of a force block, which has a wave more (the pose ahead).
+constexpr uint32_t kForceCells = 256;
+
+// 8000 box cells for a body of radius 6: a chain of latencies, not work.  All
+// of a cell's populations are loaded at once (a load per link, each waited for,
+// took 14.2 us where this takes 12.0).
 template <int Q, class ST>
-__global__ void __launch_bounds__(256) k_rigid_force(const typename ST::T* __restrict__ f, RigidArgs a) {
+__global__ void __launch_bounds__(kForceCells + 64) k_rigid_force(const typename ST::T* __restrict__ f, RigidArgs a) {
   using L = Lattice<Q>;
   using T = typename ST::T;
   __shared__ double lds[16 * 6];
@@ -107,7 +113,9 @@ __global__ void __launch_bounds__(256) k_rigid_force(const typename ST::T* __res
   __shared__ double ahead[7];  // the pose one step ahead: centre, orientation
   const RigidBody* B = a.body;
   const int tid = threadIdx.x;
-  if (tid == 0 && B->swept) {
+  const bool swept = B->swept;
+  // a wave of its own, beside the links of the others
+  if (tid == kForceCells && swept) {
     // by v and the cached omega (common_d3_geometry.wgsl get_phi3Ahead)
     const double w[3] = {B->w[0], B->w[1], B->w[2]};
     const double q[4] = {B->q[0], B->q[1], B->q[2], B->q[3]};
@@ -117,66 +125,76 @@ __global__ void __launch_bounds__(256) k_rigid_force(const typename ST::T* __res
     for (int k = 0; k < 3; k++) ahead[k] = B->c[k] + B->v[k];
     for (int k = 0; k < 4; k++) ahead[3 + k] = qa[k];
   }
-  __syncthreads();
   double fv[6] = {0, 0, 0, 0, 0, 0};
-  const uint32_t t = blockIdx.x * blockDim.x + tid;
+  const uint32_t t = blockIdx.x * kForceCells + tid;
   const uint32_t nbox = (uint32_t)a.fbox[0] * a.fbox[1] * a.fbox[2];
-  if (t < nbox) {
+  const bool mine = tid < (int)kForceCells && t < nbox;
+  double r[3] = {0, 0, 0}, fx = 0, fy = 0, fz = 0;
+  int x = 0, y = 0, z = 0;
+  bool close = false, solid_now = false;
+  double fi[Q];  // the cell's populations, unshifted: all loads at once
+  if (mine) {
     const int kx = t % a.fbox[0], ky = (t / a.fbox[0]) % a.fbox[1], kz = t / (a.fbox[0] * a.fbox[1]);
-    const int x = box_coord(B->c[0], a.half, a.fbox[0], a.nx, kx);
-    const int y = box_coord(B->c[1], a.half, a.fbox[1], a.ny, ky);
-    const int z = box_coord(B->c[2], a.half, a.fbox[2], a.nz, kz);
-    double r[3];
+    x = box_coord(B->c[0], a.half, a.fbox[0], a.nx, kx);
+    y = box_coord(B->c[1], a.half, a.fbox[1], a.ny, ky);
+    z = box_coord(B->c[2], a.half, a.fbox[2], a.nz, kz);
     body_delta(B, x, y, z, r);
-    if (len3(r[0], r[1], r[2]) <= B->rc + 2.0) {
-      const uint32_t cell = (uint32_t)((z * a.ny + y) * a.nx + x);
-      const T* blk = cell_block<ST, Q>(f, cell);
-      const uint32_t lo = cell % kLatBlock;
-      const bool solid_now = a.cls[cell] & 1;
-      const uint32_t lm = a.links[cell];
-      double fx = 0, fy = 0, fz = 0;
-      if (!solid_now && lm) {
-        double us[3];
-        body_velocity(B, x, y, z, us);
-        double rho_w = 1.0;
-        if (B->rho_w_local) {
-          rho_w = 0.0;
-          for (int i = 0; i < Q; i++) rho_w += (double)ST::load(blk + i * kLatBlock, lo) + (double)L::w[i];
-        }
+    close = len3(r[0], r[1], r[2]) <= B->rc + 2.0;
+  }
+  if (close) {
+    const uint32_t cell = (uint32_t)((z * a.ny + y) * a.nx + x);
+    const T* blk = cell_block<ST, Q>(f, cell);
+    const uint32_t lo = cell % kLatBlock;
+    solid_now = a.cls[cell] & 1;
+    const uint32_t lm = a.links[cell];
+    float g[Q];
 #pragma unroll
-        for (int i = 1; i < Q; i++) {
-          if (!((lm >> i) & 1u)) continue;
-          const double eu = L::ex[i] * us[0] + L::ey[i] * us[1] + L::ez[i] * us[2];
-          const int j = L::opp[i];
-          const double m = 2.0 * ((double)ST::load(blk + j * kLatBlock, lo) + (double)L::w[j]) +
-                           2.0 * (double)L::w[i] * rho_w * eu * 3.0;
-          fx -= L::ex[i] * m;
-          fy -= L::ey[i] * m;
-          fz -= L::ez[i] * m;
-        }
+    for (int i = 0; i < Q; i++) g[i] = ST::load(blk + i * kLatBlock, lo);
+#pragma unroll
+    for (int i = 0; i < Q; i++) fi[i] = (double)g[i] + (double)L::w[i];
+    if (!solid_now && lm) {
+      double us[3];
+      body_velocity(B, x, y, z, us);
+      double rho_w = 1.0;
+      if (B->rho_w_local) {
+        rho_w = 0.0;
+#pragma unroll
+        for (int i = 0; i < Q; i++) rho_w += fi[i];
       }
-      if (B->swept) {
-        const double ca[3] = {ahead[0], ahead[1], ahead[2]};
-        const double qa[4] = {ahead[3], ahead[4], ahead[5], ahead[6]};
-        if (solid_now != (body_phi(B, ca, qa, x, y, z) < 0.0)) {
-          double mx = 0, my = 0, mz = 0;
-          for (int i = 0; i < Q; i++) {
-            const double fi = (double)ST::load(blk + i * kLatBlock, lo) + (double)L::w[i];
-            mx += fi * L::ex[i];
-            my += fi * L::ey[i];
-            mz += fi * L::ez[i];
-          }
-          const double s = solid_now ? -1.0 : 1.0;
-          fx += s * mx;
-          fy += s * my;
-          fz += s * mz;
-        }
+#pragma unroll
+      for (int i = 1; i < Q; i++) {
+        if (!((lm >> i) & 1u)) continue;
+        const double eu = L::ex[i] * us[0] + L::ey[i] * us[1] + L::ez[i] * us[2];
+        const double m = 2.0 * fi[L::opp[i]] + 2.0 * (double)L::w[i] * rho_w * eu * 3.0;
+        fx -= L::ex[i] * m;
+        fy -= L::ey[i] * m;
+        fz -= L::ez[i] * m;
       }
-      fv[0] = fx; fv[1] = fy; fv[2] = fz;
-      fv[3] = r[1] * fz - r[2] * fy;
-      fv[4] = r[2] * fx - r[0] * fz;
-      fv[5] = r[0] * fy - r[1] * fx;
     }
+  }
+  __syncthreads();
+  if (close && swept) {
+    const double ca[3] = {ahead[0], ahead[1], ahead[2]};
+    const double qa[4] = {ahead[3], ahead[4], ahead[5], ahead[6]};
+    if (solid_now != (body_phi(B, ca, qa, x, y, z) < 0.0)) {
+      double mx = 0, my = 0, mz = 0;
+#pragma unroll
+      for (int i = 0; i < Q; i++) {
+        mx += fi[i] * L::ex[i];
+        my += fi[i] * L::ey[i];
+        mz += fi[i] * L::ez[i];
+      }
+      const double s = solid_now ? -1.0 : 1.0;
+      fx += s * mx;
+      fy += s * my;
+      fz += s * mz;
+    }
+  }
+  if (close) {
+    fv[0] = fx; fv[1] = fy; fv[2] = fz;
+    fv[3] = r[1] * fz - r[2] * fy;
+    fv[4] = r[2] * fx - r[0] * fz;
+    fv[5] = r[0] * fy - r[1] * fx;
   }
   block_sum<6>(fv, lds);
   const unsigned nblocks = gridDim.x;
@@ -191,13 +209,17 @@ __global__ void __launch_bounds__(256) k_rigid_force(const typename ST::T* __res
   // wave 0: lane l sums blocks l, l + 64, ... in order, then a fixed
   // butterfly, so the totals repeat bit for bit
   if (tid >= 64) return;
-  double tot[6];
-  for (int k = 0; k < 6; k++) {
-    double sk = 0.0;
-    for (unsigned j = tid; j < nblocks; j += 64)
-      sk += __hip_atomic_load(&a.partials[(size_t)j * 6 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    tot[k] = wave_sum(sk);
+  double tot[6] = {0, 0, 0, 0, 0, 0};
+  for (unsigned j = tid; j < nblocks; j += 64) {
+    double v[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+      v[k] = __hip_atomic_load(&a.partials[(size_t)j * 6 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 0; k < 6; k++) tot[k] += v[k];
   }
+#pragma unroll
+  for (int k = 0; k < 6; k++) tot[k] = wave_sum(tot[k]);
   if (tid == 0) {
     *a.counter = 0u;
     const unsigned long long n = *a.written;
@@ -208,52 +230,62 @@ __global__ void __launch_bounds__(256) k_rigid_force(const typename ST::T* __res
   }
 }
 
+// Half a wave a cell, a lane a direction: a lane evaluates the cell's distance
+// and one source's, where a thread a cell went through up to Q - 1 sources one
+// after the other (13.8 us for 10600 box cells, 5.1 now).
 template <int Q>
 __global__ void __launch_bounds__(256) k_rigid_classify(RigidArgs a) {
   using L = Lattice<Q>;
   const RigidBody* B = a.body;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 5;
+  const int i = threadIdx.x & 31;
   const uint32_t nbox = (uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2];
-  if (t >= nbox) return;
-  const int kx = t % a.cbox[0], ky = (t / a.cbox[0]) % a.cbox[1], kz = t / (a.cbox[0] * a.cbox[1]);
-  // the box starts below both the new centre and the previous one (c - v)
-  const int x = box_coord(fmin(B->c[0], B->c[0] - B->v[0]), a.half, a.cbox[0], a.nx, kx);
-  const int y = box_coord(fmin(B->c[1], B->c[1] - B->v[1]), a.half, a.cbox[1], a.ny, ky);
-  const int z = box_coord(fmin(B->c[2], B->c[2] - B->v[2]), a.half, a.cbox[2], a.nz, kz);
-  const uint32_t cell = (uint32_t)((z * a.ny + y) * a.nx + x);
-  double r[3];
-  body_delta(B, x, y, z, r);
-  uint8_t cl = 0;
-  uint32_t lm = 0;
-  if (len3(r[0], r[1], r[2]) <= B->rc + 2.0) {
-    const double c[3] = {B->c[0], B->c[1], B->c[2]};
-    const double q[4] = {B->q[0], B->q[1], B->q[2], B->q[3]};
-    const double phi = body_phi(B, c, q, x, y, z);
-    if (phi < 0.0) {
-      cl = 1;
-    } else if (phi < 1.75) {
+  const bool inside = t < nbox;
+  int x = 0, y = 0, z = 0;
+  bool solid = false, link = false;
+  if (inside) {
+    const int kx = t % a.cbox[0], ky = (t / a.cbox[0]) % a.cbox[1], kz = t / (a.cbox[0] * a.cbox[1]);
+    // the box starts below both the new centre and the previous one (c - v)
+    x = box_coord(fmin(B->c[0], B->c[0] - B->v[0]), a.half, a.cbox[0], a.nx, kx);
+    y = box_coord(fmin(B->c[1], B->c[1] - B->v[1]), a.half, a.cbox[1], a.ny, ky);
+    z = box_coord(fmin(B->c[2], B->c[2] - B->v[2]), a.half, a.cbox[2], a.nz, kz);
+    double r[3];
+    body_delta(B, x, y, z, r);
+    if (len3(r[0], r[1], r[2]) <= B->rc + 2.0) {
+      const double c[3] = {B->c[0], B->c[1], B->c[2]};
+      const double q[4] = {B->q[0], B->q[1], B->q[2], B->q[3]};
+      const double phi = body_phi(B, c, q, x, y, z);
+      solid = phi < 0.0;
       // a signed distance is 1-Lipschitz and a link at most sqrt(3) long, so
       // only cells this close can pull from a solid cell
-      for (int i = 1; i < Q; i++)
-        if (body_phi(B, c, q, x - L::ex[i], y - L::ey[i], z - L::ez[i]) < 0.0) lm |= 1u << i;
-      if (lm) cl = 2;
+      if (!solid && phi < 1.75 && i >= 1 && i < Q) {
+        int ex = 0, ey = 0, ez = 0;
+#pragma unroll
+        for (int k = 1; k < Q; k++)
+          if (i == k) ex = L::ex[k], ey = L::ey[k], ez = L::ez[k];
+        link = body_phi(B, c, q, x - ex, y - ey, z - ez) < 0.0;
+      }
     }
   }
-  a.cls[cell] = cl;
-  a.links[cell] = lm;
+  const uint32_t lm = (uint32_t)(__ballot(link) >> (threadIdx.x & 32));
+  if (inside && i == 0) {
+    const uint32_t cell = (uint32_t)((z * a.ny + y) * a.nx + x);
+    a.cls[cell] = solid ? 1 : (lm ? 2 : 0);
+    a.links[cell] = lm;
+  }
 }
 
 uint32_t rigid_force_blocks(const RigidArgs& a) {
-  return ((uint32_t)a.fbox[0] * a.fbox[1] * a.fbox[2] + 255) / 256;
+  return ((uint32_t)a.fbox[0] * a.fbox[1] * a.fbox[2] + kForceCells - 1) / kForceCells;
 }
 
 template <int Q>
 static hipError_t force_q(int storage, const void* f, const RigidArgs& a, hipStream_t s) {
-  const dim3 grid(rigid_force_blocks(a));
-  if (storage == kF32) hipLaunchKernelGGL((k_rigid_force<Q, StoreF32>), grid, dim3(256), 0, s, (const float*)f, a);
+  const dim3 grid(rigid_force_blocks(a)), block(kForceCells + 64);
+  if (storage == kF32) hipLaunchKernelGGL((k_rigid_force<Q, StoreF32>), grid, block, 0, s, (const float*)f, a);
   else if (storage == kF16)
-    hipLaunchKernelGGL((k_rigid_force<Q, StoreF16>), grid, dim3(256), 0, s, (const uint16_t*)f, a);
-  else hipLaunchKernelGGL((k_rigid_force<Q, StoreBF16>), grid, dim3(256), 0, s, (const uint16_t*)f, a);
+    hipLaunchKernelGGL((k_rigid_force<Q, StoreF16>), grid, block, 0, s, (const uint16_t*)f, a);
+  else hipLaunchKernelGGL((k_rigid_force<Q, StoreBF16>), grid, block, 0, s, (const uint16_t*)f, a);
   return hipGetLastError();
 }
 
@@ -262,7 +294,7 @@ hipError_t launch_rigid_force(int q, int storage, const void* f, const RigidArgs
 }
 
 hipError_t launch_rigid_classify(int q, const RigidArgs& a, hipStream_t s) {
-  const dim3 grid(((uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2] + 255) / 256);
+  const dim3 grid(((uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2] + 7) / 8);
   if (q == 19) hipLaunchKernelGGL(k_rigid_classify<19>, grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL(k_rigid_classify<27>, grid, dim3(256), 0, s, a);
   return hipGetLastError();
