@@ -446,7 +446,9 @@ PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, con
   const bool whole = (uint64_t)nx * ny % kLatBlock == 0;
   const double plane_us = q == 19 ? (general ? 5.2 : 3.5) : (general ? 7.2 : 4.8);
   const double pair_us = std::max(plane_us * best, bytes * 1.07 / 4.7e6 * (q == 19 ? 1.0 : 1.2)) * (whole ? 1.0 : 1.25);
-  const double step_us = std::max(3.8, (bytes / 6.0e6 + 2.0) * (nx % (int)kLatBlock == 0 ? 1.0 : 1.1));
+  // one by one, lattices that stay in the last-level cache or not
+  const double step_us = std::max(3.8, bytes <= 270e6 ? bytes / 7.2e6 + 2.0
+                                                      : (bytes / 6.0e6 + 2.0) * (nx % (int)kLatBlock == 0 ? 1.0 : 1.1));
   if (pair_us > 0.97 * 2.0 * step_us) return plan;
   plan.rows = rows;
   // chunk by chunk over the columns, so that neighbouring columns march the

@@ -728,6 +728,21 @@ namespace {
 
 const int kTotalsBlocks = 1024;  // max totals partial blocks
 
+// Whether the step's default launches leave both lattices in the 256 MB of
+// last-level cache between steps: ordinary loads and stores, and neighbouring
+// tiles on one XCD, in place of non-temporal access.  us a step before and
+// after, one step a launch: D3Q19 fp32 200x100x19 (60 MB) 13.0 and 10.1,
+// 200x100x78 (240 MB) 44.8 and 34.3, x88 (270 MB) 50.2 and 39.0, x98 (300 MB)
+// 54.9 and 52.1, x115 (350 MB) 63.9 and 65.4; f16 with walls 200x100x157 (240 MB)
+// 50.6 and 43.4; D2Q9 400x5208 (150 MB) 28.4 and 22.3.  Rows of whole 256-cell
+// tiles gain less (256x128x48, 240 MB: 41.8 and 34.7) and small ones nothing
+// (10 MB: f16 5.56 and 5.70; D3Q27 with walls, 60 MB: 12.5 and 13.4).
+bool cache_resident(const lbm_solve* s) {
+  const double mb = 2e-6 * lattice_elems(s->q, s->N) * s->elem;
+  const double least = s->d.nx % 256 ? 0.0 : (s->q == 27 && s->general ? 100.0 : 30.0);
+  return mb >= least && mb <= 270.0;
+}
+
 int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, int by, int flags,
                 lbm_solve** out) {
   if (!out) return fail(LBM_E_INVALID, "null output handle");
@@ -754,6 +769,10 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
     s->nt = (flags >> 1) & 1;
     s->lin = (flags >> 2) & 1;
     s->occ = (flags >> 4) & 15;
+    if (!arena && !desc->diffuse && cache_resident(s)) {
+      s->nt = 0;
+      s->swz = 1;
+    }
   }
   // launches of several steps (a pool member's steps are the batched kernel's)
   if (!arena && !desc->diffuse) {
@@ -1394,6 +1413,12 @@ int lbm_rigid_attach(lbm_solve* s, const lbm_rigid_body* b) {
   int rc = LBM_OK;
   if (!s->cls && (rc = dalloc(s, &s->cls, s->N))) return rc;
   if (!s->links && (rc = dalloc(s, &s->links, (size_t)s->N * 4))) return rc;
+  if (!s->tuned) {
+    // the rigid step keeps non-temporal access (192x72x72, 151 MB: 31.7 us a
+    // step, cache-resident launches 33.8)
+    s->nt = 1;
+    s->swz = 0;
+  }
   if (!s->rigid) {
     HIPCHK(hipMalloc((void**)&s->rigid, sizeof(RigidBody)));
     HIPCHK(hipMalloc((void**)&s->rigid_counter, 16));
