@@ -230,45 +230,60 @@ __global__ void __launch_bounds__(kForceCells + 64) k_rigid_force(const typename
   }
 }
 
-// Half a wave a cell, a lane a direction: a lane evaluates the cell's distance
-// and one source's, where a thread a cell went through up to Q - 1 sources one
-// after the other (13.8 us for 10600 box cells, 5.1 now).
-template <int Q>
+// Half a wave evaluates a cell's links, a lane a direction, where a thread a
+// cell goes through up to Q - 1 sources one after the other.  A small box has
+// half a wave per cell from the start (WIDE false); in a large one, most of
+// whose cells are far from the surface, a lane first takes each cell's own
+// distance and the half waves then go through the cells next to it.
+template <int Q, bool WIDE>
 __global__ void __launch_bounds__(256) k_rigid_classify(RigidArgs a) {
   using L = Lattice<Q>;
   const RigidBody* B = a.body;
-  const uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 5;
-  const int i = threadIdx.x & 31;
+  const uint32_t t = WIDE ? blockIdx.x * blockDim.x + threadIdx.x : blockIdx.x * (blockDim.x >> 5) + (threadIdx.x >> 5);
+  const int i = threadIdx.x & 31, half = threadIdx.x & 32;
   const uint32_t nbox = (uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2];
   const bool inside = t < nbox;
+  const double c[3] = {B->c[0], B->c[1], B->c[2]};
+  const double q[4] = {B->q[0], B->q[1], B->q[2], B->q[3]};
   int x = 0, y = 0, z = 0;
-  bool solid = false, link = false;
+  bool solid = false, near = false;
   if (inside) {
     const int kx = t % a.cbox[0], ky = (t / a.cbox[0]) % a.cbox[1], kz = t / (a.cbox[0] * a.cbox[1]);
     // the box starts below both the new centre and the previous one (c - v)
-    x = box_coord(fmin(B->c[0], B->c[0] - B->v[0]), a.half, a.cbox[0], a.nx, kx);
-    y = box_coord(fmin(B->c[1], B->c[1] - B->v[1]), a.half, a.cbox[1], a.ny, ky);
-    z = box_coord(fmin(B->c[2], B->c[2] - B->v[2]), a.half, a.cbox[2], a.nz, kz);
+    x = box_coord(fmin(c[0], c[0] - B->v[0]), a.half, a.cbox[0], a.nx, kx);
+    y = box_coord(fmin(c[1], c[1] - B->v[1]), a.half, a.cbox[1], a.ny, ky);
+    z = box_coord(fmin(c[2], c[2] - B->v[2]), a.half, a.cbox[2], a.nz, kz);
     double r[3];
     body_delta(B, x, y, z, r);
     if (len3(r[0], r[1], r[2]) <= B->rc + 2.0) {
-      const double c[3] = {B->c[0], B->c[1], B->c[2]};
-      const double q[4] = {B->q[0], B->q[1], B->q[2], B->q[3]};
       const double phi = body_phi(B, c, q, x, y, z);
       solid = phi < 0.0;
       // a signed distance is 1-Lipschitz and a link at most sqrt(3) long, so
       // only cells this close can pull from a solid cell
-      if (!solid && phi < 1.75 && i >= 1 && i < Q) {
-        int ex = 0, ey = 0, ez = 0;
-#pragma unroll
-        for (int k = 1; k < Q; k++)
-          if (i == k) ex = L::ex[k], ey = L::ey[k], ez = L::ez[k];
-        link = body_phi(B, c, q, x - ex, y - ey, z - ez) < 0.0;
-      }
+      near = !solid && phi < 1.75;
     }
   }
-  const uint32_t lm = (uint32_t)(__ballot(link) >> (threadIdx.x & 32));
-  if (inside && i == 0) {
+  int ex = 0, ey = 0, ez = 0;  // this lane's direction
+#pragma unroll
+  for (int k = 1; k < Q; k++)
+    if (i == k) ex = L::ex[k], ey = L::ey[k], ez = L::ez[k];
+  const bool moving = i >= 1 && i < Q;
+  // the half wave's links of the cell (sx, sy, sz)
+  auto links_of = [&](bool wanted, int sx, int sy, int sz) {
+    const bool link = wanted && moving && body_phi(B, c, q, sx - ex, sy - ey, sz - ez) < 0.0;
+    return (uint32_t)(__ballot(link) >> half);
+  };
+  uint32_t lm = 0;
+  if constexpr (WIDE) {
+    for (uint32_t todo = (uint32_t)(__ballot(near) >> half); todo; todo &= todo - 1) {
+      const int lane = __ffs(todo) - 1;
+      const uint32_t m = links_of(true, __shfl(x, lane, 32), __shfl(y, lane, 32), __shfl(z, lane, 32));
+      if (i == lane) lm = m;
+    }
+  } else {
+    lm = links_of(near, x, y, z);
+  }
+  if (inside && (WIDE || i == 0)) {
     const uint32_t cell = (uint32_t)((z * a.ny + y) * a.nx + x);
     a.cls[cell] = solid ? 1 : (lm ? 2 : 0);
     a.links[cell] = lm;
@@ -293,11 +308,24 @@ hipError_t launch_rigid_force(int q, int storage, const void* f, const RigidArgs
   return q == 19 ? force_q<19>(storage, f, a, s) : force_q<27>(storage, f, a, s);
 }
 
-hipError_t launch_rigid_classify(int q, const RigidArgs& a, hipStream_t s) {
-  const dim3 grid(((uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2] + 7) / 8);
-  if (q == 19) hipLaunchKernelGGL(k_rigid_classify<19>, grid, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(k_rigid_classify<27>, grid, dim3(256), 0, s, a);
+// Largest box, in cells, that takes half a wave a cell.  Beyond, most of its
+// cells need one distance only, and 32 threads for each of 2^27 cells would be
+// more than a launch's 2^32.  us, half a wave a cell and WIDE (a thread a cell
+// that also goes through its own links, before either): 14k cells 6.8, 12.0
+// (15.8); 22k 9.6, 11.0 (16.0); 33k 13.4, 10.3 (15.7); 64k 21.6, 11.4 (14.2);
+// 373k 108, 22.4 (33.6); 2.3M 634, 66 (132).
+constexpr uint32_t kSmallBox = 24000;
+
+template <int Q>
+static hipError_t classify_q(const RigidArgs& a, hipStream_t s) {
+  const uint32_t nbox = (uint32_t)a.cbox[0] * a.cbox[1] * a.cbox[2];
+  if (nbox <= kSmallBox) hipLaunchKernelGGL((k_rigid_classify<Q, false>), dim3((nbox + 7) / 8), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((k_rigid_classify<Q, true>), dim3((nbox + 255) / 256), dim3(256), 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_rigid_classify(int q, const RigidArgs& a, hipStream_t s) {
+  return q == 19 ? classify_q<19>(a, s) : classify_q<27>(a, s);
 }
 
 }  // namespace lbm
