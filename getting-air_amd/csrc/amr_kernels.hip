@@ -1481,7 +1481,9 @@ struct OpExplode {
                         int linear, int dirs, const PoolForce* force, hipStream_t s) {
     // about 2^20 threads: every direction its own thread for a small ring,
     // all Q in one thread for a ring of a million cells
-    const int split = (int)std::min<uint64_t>(Q, std::max<uint64_t>(1, ((1u << 20) + nring - 1) / nring));
+    // (no ring: the force pass alone)
+    const uint32_t cells = std::max(nring, 1u);
+    const int split = (int)std::min<uint64_t>(Q, std::max<uint64_t>(1, ((1u << 20) + cells - 1) / cells));
     const int per = dirs > 0 ? std::min(dirs, Q) : (Q + split - 1) / split;
     const uint32_t nblocks = grid_for(nring).x, groups = (Q + per - 1) / per;
     auto go = [&](auto PP, auto F, uint32_t extra) {
@@ -1583,9 +1585,8 @@ hipError_t launch_reflux(int q, const float* gct, float* gct1, float* mac, const
 
 hipError_t launch_explode(int q, const ParentRef& parent, float* gp, const PoolGeom& g, const SurfacePlan& plan,
                           uint32_t nring, int linear, int dirs, const PoolForce* force, hipStream_t s) {
-  // a body always lies in some tile
-  if (force && (nring == 0 || force->nactive <= 0)) return hipErrorInvalidConfiguration;
-  if (nring == 0) return hipSuccess;
+  // a body outside the grid lies in no tile: its force pass leaves zeros
+  if (nring == 0 && !force) return hipSuccess;
   return dispatch_q_rb<OpExplode>(q, g.rb, parent, gp, g, plan, nring, linear, dirs, force, s);
 }
 
