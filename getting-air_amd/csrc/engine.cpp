@@ -128,6 +128,7 @@ struct lbm_solve {
   int bx = 64, by = 1, swz = 1, nt = 0;
   int occ = 0;                      // waves-per-SIMD cap of the step launches (0: none)
   int lin = 0;                      // linear tiles (blocks of consecutive cells)
+  bool cached_default = false;      // nt and swz are cache_resident's, not a caller's or the autotuner's
   int force_pending = 0;            // steps of the last launch whose forces are not yet summed
   int pair_rows = 0;                // two-step launches: rows of a block (0: none),
   PairBlock* pair_blocks = nullptr; // and the blocks
@@ -648,6 +649,7 @@ int autotune(lbm_solve* s) {
   }
   s->bx = bestv.bx; s->by = bestv.by; s->swz = bestv.swz; s->nt = bestv.nt; s->occ = bestv.occ;
   s->lin = bestv.lin;
+  s->cached_default = false;
   s->tuned = true;
   return build_force_slots(s);
 }
@@ -772,6 +774,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
     if (!arena && !desc->diffuse && cache_resident(s)) {
       s->nt = 0;
       s->swz = 1;
+      s->cached_default = true;
     }
   }
   // launches of several steps (a pool member's steps are the batched kernel's)
@@ -1280,6 +1283,7 @@ int lbm_set_tile(lbm_solve* s, int32_t block_x, int32_t block_y, int32_t flags) 
   s->nt = (flags >> 1) & 1;
   s->lin = (flags >> 2) & 1;
   s->occ = occ;
+  s->cached_default = false;
   s->tuned = true;
   s->pair_rows = 0;  // the caller asks for this tile's launches
   s->multi = MultiPlan{};
@@ -1413,11 +1417,12 @@ int lbm_rigid_attach(lbm_solve* s, const lbm_rigid_body* b) {
   int rc = LBM_OK;
   if (!s->cls && (rc = dalloc(s, &s->cls, s->N))) return rc;
   if (!s->links && (rc = dalloc(s, &s->links, (size_t)s->N * 4))) return rc;
-  if (!s->tuned) {
+  if (s->cached_default) {
     // the rigid step keeps non-temporal access (192x72x72, 151 MB: 31.7 us a
     // step, cache-resident launches 33.8)
     s->nt = 1;
     s->swz = 0;
+    s->cached_default = false;
   }
   if (!s->rigid) {
     HIPCHK(hipMalloc((void**)&s->rigid, sizeof(RigidBody)));
