@@ -246,9 +246,10 @@ struct PairArgs {
   int32_t finalize_prev;  // block 0 appends the previous launch's records (StepArgs::prev)
 };
 // The blocks for a grid whose boundary cells (ascending) are given; rows 0
-// where one-step launches are the faster ones or the pair kernel does not
-// take the grid.
-PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary);
+// where the pair kernel does not take the grid or, unless `always`, one-step
+// launches are the faster ones.
+PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary,
+                   bool always);
 hipError_t launch_step_pair(int q, bool general, const void* fin, void* fout, const StepArgs& a, const PairArgs& p,
                             hipStream_t s);
 // Several D2Q9 steps in one launch (dense_multi.hip), on the bounce-back

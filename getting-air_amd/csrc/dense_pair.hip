@@ -383,14 +383,15 @@ static constexpr size_t pair_lds() {
   return (size_t)2 * lds_slots<Q>() * (pair_rows<Q>() + 2) * kPitch * sizeof(float);
 }
 
-PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary) {
+PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, const std::vector<uint32_t>& boundary,
+                   bool always) {
   PairPlan plan;
   const double cells = (double)nx * ny * nz, bytes = cells * 2 * q * 4;
   // the kernel's 32-bit in-plane byte offsets and, with walls or a body, its
   // 32-bit lattice ones
   if (q == 9 || storage != kF32 || (double)nx * ny * q * 4 >= 4.0e9 || (general && bytes / 2 >= 4.0e9)) return plan;
   // lanes past the end of a row idle: a narrow last column costs a whole one
-  if (nx < 0.7 * kTileX * ((nx + kTileX - 1) / kTileX)) return plan;
+  if (!always && nx < 0.7 * kTileX * ((nx + kTileX - 1) / kTileX)) return plan;
   const int most = q == 19 ? pair_rows<19>() : pair_rows<27>();
   const int nty = (ny + most - 1) / most, rows = (ny + nty - 1) / nty, ntx = (nx + kTileX - 1) / kTileX;
   const int cols = ntx * nty;
@@ -449,7 +450,7 @@ PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, con
   // one by one, lattices that stay in the last-level cache or not
   const double step_us = std::max(3.8, bytes <= 270e6 ? bytes / 7.2e6 + 2.0
                                                       : (bytes / 6.0e6 + 2.0) * (nx % (int)kLatBlock == 0 ? 1.0 : 1.1));
-  if (pair_us > 0.97 * 2.0 * step_us) return plan;
+  if (!always && pair_us > 0.97 * 2.0 * step_us) return plan;
   plan.rows = rows;
   // chunk by chunk over the columns, so that neighbouring columns march the
   // same planes at the same time on one XCD

@@ -349,9 +349,10 @@ int build_boundary_slots(lbm_solve* s) {
   return LBM_OK;
 }
 
-// The two-step launch's blocks, where pairs are the faster form.
-int build_pair_blocks(lbm_solve* s) {
-  const PairPlan plan = pair_plan(s->q, s->storage, s->general, s->d.nx, s->d.ny, s->d.nz, s->boundary);
+// The two-step launch's blocks, where pairs are the faster form (`always`:
+// wherever the kernel takes the grid).
+int build_pair_blocks(lbm_solve* s, bool always) {
+  const PairPlan plan = pair_plan(s->q, s->storage, s->general, s->d.nx, s->d.ny, s->d.nz, s->boundary, always);
   if (plan.rows <= 0) return LBM_OK;
   const size_t bytes = plan.blocks.size() * sizeof(PairBlock);
   int rc = dalloc(s, &s->pair_blocks, bytes);
@@ -820,7 +821,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
       return rc;
     }
   }
-  if (!arena && !desc->diffuse && (rc = build_pair_blocks(s))) {
+  if (!arena && !desc->diffuse && (rc = build_pair_blocks(s, false))) {
     release(s);
     return rc;
   }
@@ -1289,6 +1290,46 @@ int lbm_set_tile(lbm_solve* s, int32_t block_x, int32_t block_y, int32_t flags) 
   s->multi = MultiPlan{};
   int rc = build_force_slots(s);
   if (rc) return rc;
+  return prepare_graphs(s);
+}
+
+int lbm_launch_steps(lbm_solve* s, int32_t* steps) {
+  if (!s || !steps) return fail(LBM_E_INVALID, "null argument");
+  *steps = launch_steps(s);
+  return LBM_OK;
+}
+
+int lbm_set_launch_steps(lbm_solve* s, int32_t steps) {
+  if (!s) return fail(LBM_E_INVALID, "null solve");
+  if (steps < 0 || steps > kMaxLaunchSteps) return fail(LBM_E_INVALID, "%d steps a launch: 0 to %d", steps, kMaxLaunchSteps);
+  const MultiPlan plan = s->d.diffuse ? MultiPlan{} : multi_plan(s->q, s->d.nx, s->d.ny);
+  if (steps > 1) {
+    if (s->d.diffuse || s->rigid)
+      return fail(LBM_E_REFUSED, "a %s takes one step a launch", s->rigid ? "moving body" : "diffuse coupling");
+    if (s->dim == 2 && steps > plan.steps)
+      return fail(LBM_E_REFUSED, "%d steps a launch on %dx%d: at most %d", steps, s->d.nx, s->d.ny, std::max(1, plan.steps));
+    if (s->dim == 3 && (steps != 2 || s->storage != LBM_STORE_F32))
+      return fail(LBM_E_REFUSED, "%d steps a launch: 3D lattices take 2 at most, in fp32 storage", steps);
+  }
+  HIPCHK(hipStreamSynchronize(s->stream));
+  drop_graphs(s);
+  if (s->pair_blocks) {
+    HIPCHK(hipFree(s->pair_blocks));
+    s->pair_blocks = nullptr;
+    s->bytes -= (size_t)s->pair_nblocks * sizeof(PairBlock);
+  }
+  s->pair_rows = 0;
+  s->multi = MultiPlan{};
+  if (s->dim == 2 && steps != 1) {
+    s->multi = plan;
+    if (steps > 1) s->multi.steps = steps;
+  }
+  if (s->dim == 3 && steps != 1 && !s->d.diffuse) {
+    int rc = build_pair_blocks(s, steps == 2);
+    if (rc) return rc;
+    if (steps == 2 && !s->pair_rows)
+      return fail(LBM_E_REFUSED, "the two-step kernel does not take %dx%dx%d", s->d.nx, s->d.ny, s->d.nz);
+  }
   return prepare_graphs(s);
 }
 

@@ -22,7 +22,7 @@ EXPORTS = (
     "lbm_solve_destroy", "lbm_upload_macro", "lbm_upload_f", "lbm_read_f", "lbm_step",
     "lbm_step_timed", "lbm_sync", "lbm_read_macro", "lbm_read_forces", "lbm_read_totals",
     "lbm_read_classes", "lbm_solve_info", "lbm_set_tile", "lbm_time_step_kernel",
-    "lbm_probe_copy_bandwidth", "lbm_state_size", "lbm_save_state", "lbm_load_state",
+    "lbm_launch_steps", "lbm_set_launch_steps", "lbm_probe_copy_bandwidth", "lbm_state_size", "lbm_save_state", "lbm_load_state",
     "lbm_amr_create", "lbm_amr_destroy", "lbm_amr_upload_topology", "lbm_amr_read_topology",
     "lbm_amr_upload_macro", "lbm_amr_step", "lbm_amr_manage_now", "lbm_amr_read_macro",
     "lbm_amr_read_pool_macro", "lbm_amr_read_f", "lbm_amr_read_criterion", "lbm_amr_read_active",
@@ -174,6 +174,8 @@ def load():
                                        ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32),
                                        ctypes.POINTER(ctypes.c_int64)]
         lib.lbm_set_tile.argtypes = [P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]
+        lib.lbm_launch_steps.argtypes = [P, ctypes.POINTER(ctypes.c_int32)]
+        lib.lbm_set_launch_steps.argtypes = [P, ctypes.c_int32]
         lib.lbm_time_step_kernel.argtypes = [P, ctypes.c_int32, ctypes.POINTER(ctypes.c_double)]
         lib.lbm_state_size.argtypes = [P, ctypes.POINTER(ctypes.c_size_t)]
         lib.lbm_save_state.argtypes = [P, P, ctypes.c_size_t]
@@ -388,8 +390,19 @@ class Solve:
         _check(self.lib.lbm_load_state(self.h, b.ctypes.data, b.size))
 
     def set_tile(self, bx, by, flags):
-        """flags: bit 0 XCD swizzle, bit 1 non-temporal, bit 2 linear tiles, bits 4-7 waves-per-SIMD cap."""
+        """flags: bit 0 XCD swizzle, bit 1 non-temporal, bit 2 linear tiles, bits 4-7 waves-per-SIMD cap.
+        Pins the solve to one-step launches."""
         _check(self.lib.lbm_set_tile(self.h, int(bx), int(by), int(flags)))
+
+    def launch_steps(self):
+        """Steps that one kernel launch of step() advances."""
+        n = ctypes.c_int32()
+        _check(self.lib.lbm_launch_steps(self.h, ctypes.byref(n)))
+        return n.value
+
+    def set_launch_steps(self, n):
+        """0: the engine's choice; 1: one-step launches; more where the kernels take the solve."""
+        _check(self.lib.lbm_set_launch_steps(self.h, int(n)))
 
     def time_step_kernel(self, n):
         """Mean device milliseconds of one fused stream-collide launch."""

@@ -204,8 +204,20 @@ int lbm_solve_info(lbm_solve* s, int64_t* step, int32_t* block_x, int32_t* block
  * selects non-temporal loads and stores, bit 2 makes tiles linear (a block
  * steps block_x * block_y consecutive cells of the x-fastest index instead of
  * a block_x by block_y patch of one z plane), bits 4-7 cap residency at that
- * many waves per SIMD (0: no cap; 4 is available for every shape). */
+ * many waves per SIMD (0: no cap; 4 is available for every shape).  The tile
+ * is that of the one-step kernel, and setting it pins the solve to launches of
+ * one step (lbm_set_launch_steps(s, 0) gives the engine its choice back). */
 int lbm_set_tile(lbm_solve* s, int32_t block_x, int32_t block_y, int32_t flags);
+
+/* Steps that one kernel launch of lbm_step advances (a remainder takes a
+ * shorter launch).  The engine chooses by lattice, grid and storage: 1, 2
+ * (fp32 D3Q19 and D3Q27) or up to 8 (D2Q9); moving bodies, the diffuse
+ * coupling and 16-bit 3D storage take 1.  Results do not depend on it. */
+int lbm_launch_steps(lbm_solve* s, int32_t* steps);
+/* Overrides that choice: 1 for one-step launches, more where the kernels take
+ * the solve (LBM_E_REFUSED otherwise): 2 in fp32 3D, in 2D at most the
+ * engine's own number; 0 returns to the engine's choice. */
+int lbm_set_launch_steps(lbm_solve* s, int32_t steps);
 
 /* Measurement hook, no counterpart in the reference (its spike page times
  * passes with timestamp queries, main-3d-spike.js:229-286): launches the
