@@ -468,10 +468,24 @@ int launch_steps(const lbm_solve* s) {
   return s->multi.shape && !s->rigid ? s->multi.steps : 1;
 }
 
-// A launch of `steps` steps, launch_steps or (2D, or a single step) fewer.
+// The longest remainder of a call (steps that do not fill a launch) that goes
+// as one-step launches; beyond, in 2D, it is one shorter launch.  us for one
+// and two D2Q9 steps, one-step launches and a shorter one of the grid's tile,
+// plain periodic: fp32 64^2 3.3, 6.3 and 3.5, 3.4; 352^2 3.6, 6.7 and 4.9, 5.7;
+// 960x480 7.1, 12.9 and 8.8, 10.8; 4096x2048 109, 209 and 153, 177; f16 960x480
+// 5.7, 10.9 and 7.8, 10.1; 4096x2048 69, 122 and 117, 143, where three take 176
+// and 171.  Two steps with body and sponge: f16 2304x1152 49.6 and 48.3,
+// 2896x1448 67.4 and 71.1; fp32 4096x2048 230 and 198, but with rows that are
+// not whole layout blocks 5000x3000 400 and 405.
+int single_steps(const lbm_solve* s) {
+  const bool large = s->multi.shape == kMultiWide && s->N >= (1u << 22);
+  return large && (s->elem == 2 || s->d.nx % (int)kLatBlock != 0) ? 2 : 1;
+}
+
+// A launch of `steps` steps, launch_steps or (2D) fewer.
 int enqueue_launch(lbm_solve* s, int steps, bool write_mac, bool finalize_prev) {
-  if (s->multi.shape) return enqueue_multi(s, steps, write_mac, finalize_prev);
-  return steps == 2 ? enqueue_pair(s, write_mac, finalize_prev) : enqueue_step(s, write_mac, finalize_prev);
+  if (steps == 1) return enqueue_step(s, write_mac, finalize_prev);
+  return s->multi.shape ? enqueue_multi(s, steps, write_mac, finalize_prev) : enqueue_pair(s, write_mac, finalize_prev);
 }
 
 // Appends the force records of the last enqueued launch.
@@ -1124,7 +1138,12 @@ int lbm_step(lbm_solve* s, int32_t n) {
     // eagerly (so that every chunk follows a launch of its own kind, whose
     // forces its first launch sums), captured chunks, single launches, the
     // last of them writing the macroscopic field.
-    if (n % per) rc = enqueue_launch(s, n % per, n < per, false);
+    const int rest = n % per;
+    if (rest > single_steps(s)) {
+      rc = enqueue_launch(s, rest, n < per, false);
+    } else {
+      for (int k = 0; k < rest && rc == LBM_OK; k++) rc = enqueue_step(s, n < per && k == rest - 1, k > 0);
+    }
     int left = n / per;
     bool first = true;
     while (left > 0 && rc == LBM_OK) {
