@@ -36,7 +36,9 @@ from pylbm import scenarios as sc  # noqa: E402
 
 METRIC = "D3Q19 MLUPS & % HBM peak, fp32 vs fp16-store; solves/s + p99 latency served"
 HBM_PEAK_GBS = 8000.0
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_d3q19_sphere_256x128x128.json")
+# measured HBM bytes of a launch, by its steps
+TRAFFIC_FILES = {n: os.path.join(ROOT, "profiles", "traffic_%sd3q19_sphere_256x128x128.json" % p)
+                 for n, p in ((1, ""), (2, "pair_"))}
 
 
 def measure(storage, steps, warmup, kernel_reps, periodic=False, tile=None):
@@ -59,6 +61,11 @@ def measure(storage, steps, warmup, kernel_reps, periodic=False, tile=None):
         t1 = time.perf_counter()
         forces = s.read_forces(steps)
         kernel_ms = s.time_step_kernel(kernel_reps)
+        per = s.launch_steps()
+        one_ms = kernel_ms
+        if per > 1:
+            s.set_launch_steps(1)
+            one_ms = s.time_step_kernel(kernel_reps)
         info = s.info()
         ncells = s.ncells
     secs = t1 - t0
@@ -71,7 +78,13 @@ def measure(storage, steps, warmup, kernel_reps, periodic=False, tile=None):
     return {
         "mlups": ncells * steps / secs / 1e6,
         "ms_per_step": secs * 1e3 / steps,
+        # the kernel the run launches; a launch of several steps reads and
+        # writes the lattice once
+        "kernel": "k_step%s<%d, Store%s, %s>" % ("_pair" if per > 1 else "", q, storage.upper(),
+                                                 "periodic" if periodic else "general"),
+        "steps_per_launch": per,
         "kernel_ms": kernel_ms,
+        "one_step_kernel_ms": one_ms,
         "achieved_gbs": achieved,
         "bytes_per_launch": bytes_per_launch,
         "ncells": ncells,
@@ -651,8 +664,9 @@ def main():
         print("turbulence: %s" % json.dumps(extra_turb), file=sys.stderr, flush=True)
 
     traffic = None
-    if os.path.exists(TRAFFIC_FILE):
-        with open(TRAFFIC_FILE) as fh:
+    traffic_file = TRAFFIC_FILES[main_run["steps_per_launch"]]
+    if os.path.exists(traffic_file):
+        with open(traffic_file) as fh:
             traffic = json.load(fh).get("hbm_bytes_per_launch")
 
     cpu = None
@@ -682,8 +696,13 @@ def main():
         "pct_hbm_peak": round(100.0 * achieved / HBM_PEAK_GBS, 2),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_step<19, StoreF32, general>", "kernel_ms": round(main_run["kernel_ms"], 5),
+                     "kernel": main_run["kernel"], "kernel_ms": round(main_run["kernel_ms"], 5),
+                     "steps_per_launch": main_run["steps_per_launch"],
                      "bytes_per_launch": main_run["bytes_per_launch"]},
+        # the same solve's one-step launch (odd steps, and every step where
+        # launches of several do not apply)
+        "one_step_kernel": {"kernel_ms": round(main_run["one_step_kernel_ms"], 5),
+                            "achieved_gbs": round(main_run["bytes_per_launch"] / main_run["one_step_kernel_ms"] / 1e6, 1)},
         "cpu_baseline": cpu,
         "drag_cd_last1000": main_run["cd_last1000"],
         "copy_probe_gbs": round(copy_gbs, 1),
@@ -691,8 +710,11 @@ def main():
     }
     for k, v in extra.items():
         out[k] = {"mlups": round(v["mlups"], 1), "speedup_vs_f32": round(v["speedup_vs_f32"], 3),
-                  "kernel_speedup_vs_f32": round(main_run["kernel_ms"] / v["kernel_ms"], 3),
-                  "kernel_ms": round(v["kernel_ms"], 5), "achieved_gbs": round(v["achieved_gbs"], 1),
+                  # per step
+                  "kernel_speedup_vs_f32": round(main_run["kernel_ms"] / main_run["steps_per_launch"] /
+                                                 (v["kernel_ms"] / v["steps_per_launch"]), 3),
+                  "steps_per_launch": v["steps_per_launch"], "kernel_ms": round(v["kernel_ms"], 5),
+                  "achieved_gbs": round(v["achieved_gbs"], 1),
                   "pct_hbm_peak": round(100.0 * v["achieved_gbs"] / HBM_PEAK_GBS, 2),
                   "cd_last1000": v["cd_last1000"],
                   "drag_dev_vs_f32_pct": (100.0 * (v["cd_last1000"] / main_run["cd_last1000"] - 1.0)

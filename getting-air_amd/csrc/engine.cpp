@@ -426,18 +426,30 @@ int enqueue_step(lbm_solve* s, bool write_mac, bool finalize_prev) {
   return LBM_OK;
 }
 
-// Two steps in one launch; the lattice parity flips once.
-int enqueue_pair(lbm_solve* s, bool write_mac, bool finalize_prev) {
-  StepArgs a = step_args(s, write_mac, true);
-  a.finalize_prev = finalize_prev && a.boundary ? 1 : 0;
-  a.prev = a.boundary ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
+// The launches of several steps from the current lattice into the other one;
+// the lattice parity, which flips once, is the caller's.
+hipError_t launch_pair(lbm_solve* s, const StepArgs& a) {
   PairArgs p{};
   p.blocks = s->pair_blocks;
   p.nblocks = s->pair_nblocks;
   p.rows = s->pair_rows;
   p.force2 = a.boundary ? force_set(s, s->parity, 1) : nullptr;
   p.finalize_prev = a.finalize_prev;
-  hipError_t e = launch_step_pair(s->q, s->general, s->f[s->parity], s->f[1 - s->parity], a, p, s->stream);
+  return launch_step_pair(s->q, s->general, s->f[s->parity], s->f[1 - s->parity], a, p, s->stream);
+}
+hipError_t launch_multi(lbm_solve* s, const StepArgs& a, int steps) {
+  MultiArgs p{};
+  p.steps = steps;
+  p.force_stride = force_stride(s);
+  return launch_step_multi(s->storage, s->multi.shape, s->general, s->f[s->parity], s->f[1 - s->parity], a, p, s->stream);
+}
+
+// Two steps in one launch.
+int enqueue_pair(lbm_solve* s, bool write_mac, bool finalize_prev) {
+  StepArgs a = step_args(s, write_mac, true);
+  a.finalize_prev = finalize_prev && a.boundary ? 1 : 0;
+  a.prev = a.boundary ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
+  hipError_t e = launch_pair(s, a);
   if (e != hipSuccess) return hip_fail(e, "two-step kernel launch");
   s->force_pending = a.boundary ? 2 : 0;
   s->parity ^= 1;
@@ -450,11 +462,7 @@ int enqueue_multi(lbm_solve* s, int steps, bool write_mac, bool finalize_prev) {
   StepArgs a = step_args(s, write_mac, true);
   a.finalize_prev = finalize_prev && a.boundary ? 1 : 0;
   a.prev = a.boundary ? force_sum(s, 1 - s->parity, s->force_pending) : ForceSum{};
-  MultiArgs p{};
-  p.steps = steps;
-  p.force_stride = force_stride(s);
-  hipError_t e = launch_step_multi(s->storage, s->multi.shape, s->general, s->f[s->parity], s->f[1 - s->parity], a, p,
-                                   s->stream);
+  hipError_t e = launch_multi(s, a, steps);
   if (e != hipSuccess) return hip_fail(e, "multi-step kernel launch");
   s->force_pending = a.boundary ? steps : 0;
   s->parity ^= 1;
@@ -1272,15 +1280,18 @@ int lbm_time_step_kernel(lbm_solve* s, int32_t n, double* ms_per_launch) {
     int rc = autotune(s);
     if (rc) return rc;
   }
-  const void* fin = s->f[s->parity];
-  void* fout = s->f[1 - s->parity];
-  StepArgs a = step_args(s, false, true);
-  HIPCHK(launch_step(s->q, s->storage, s->general, s->nt, s->occ, fin, fout, a, s->bx, s->by, s->stream,
-                     s->d.diffuse != 0));
+  // the launches that lbm_step takes
+  const StepArgs a = step_args(s, false, true);
+  const int per = launch_steps(s);
+  auto launch = [&] {
+    if (per == 1)
+      return launch_step(s->q, s->storage, s->general, s->nt, s->occ, s->f[s->parity], s->f[1 - s->parity], a, s->bx,
+                         s->by, s->stream, s->d.diffuse != 0);
+    return s->multi.shape ? launch_multi(s, a, per) : launch_pair(s, a);
+  };
+  HIPCHK(launch());
   HIPCHK(hipEventRecord(s->ev0, s->stream));
-  for (int r = 0; r < n; r++)
-    HIPCHK(launch_step(s->q, s->storage, s->general, s->nt, s->occ, fin, fout, a, s->bx, s->by, s->stream,
-                     s->d.diffuse != 0));
+  for (int r = 0; r < n; r++) HIPCHK(launch());
   HIPCHK(hipEventRecord(s->ev1, s->stream));
   HIPCHK(hipEventSynchronize(s->ev1));
   float t = 0.f;

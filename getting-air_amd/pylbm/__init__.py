@@ -405,7 +405,7 @@ class Solve:
         _check(self.lib.lbm_set_launch_steps(self.h, int(n)))
 
     def time_step_kernel(self, n):
-        """Mean device milliseconds of one fused stream-collide launch."""
+        """Mean device milliseconds of one fused stream-collide launch, of launch_steps() steps."""
         ms = ctypes.c_double()
         _check(self.lib.lbm_time_step_kernel(self.h, int(n), ctypes.byref(ms)))
         return ms.value

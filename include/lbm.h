@@ -68,7 +68,9 @@ typedef struct lbm_desc {
   lbm_body body;        /* pinned body with halfway bounce-back               */
   int32_t solid_eq;     /* SOLID_EQ: hold the body interior at feq(1, 0)      */
   int32_t storage;      /* LBM_STORE_*                                        */
-  int32_t autotune;     /* 1: time candidate tile shapes on first step        */
+  int32_t autotune;     /* 1: time candidate tile shapes of the one-step kernel
+                         * when the state is set (also where most launches take
+                         * several steps and it takes the remainders)         */
   int32_t diffuse;      /* the body's coupling.  0: halfway bounce-back with
                          * momentum exchange (?bounceback, USE_BOUNCEBACK).
                          * 1: the diffuse penalty coupling, the reference's
@@ -221,10 +223,10 @@ int lbm_set_launch_steps(lbm_solve* s, int32_t steps);
 
 /* Measurement hook, no counterpart in the reference (its spike page times
  * passes with timestamp queries, main-3d-spike.js:229-286): launches the
- * fused stream-collide kernel n times from the current lattice into the other
- * one without swapping (the state does not advance) and returns the mean
- * device time of one launch in milliseconds, bracketed by HIP events on the
- * solve's stream. */
+ * fused stream-collide kernel that lbm_step takes, lbm_launch_steps steps of
+ * it, n times from the current lattice into the other one without swapping
+ * (the state does not advance) and returns the mean device time of one launch
+ * in milliseconds, bracketed by HIP events on the solve's stream. */
 int lbm_time_step_kernel(lbm_solve* s, int32_t n, double* ms_per_launch);
 
 /* Measurement hook, no counterpart in the reference: a 16-byte streaming
