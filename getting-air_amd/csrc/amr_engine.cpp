@@ -651,6 +651,13 @@ int manage(lbm_amr* a) {
   return LBM_OK;
 }
 
+// Both lattices and the macroscopic field of the active tiles of every level, MB.
+double tiles_mb(const lbm_amr* a) {
+  double n = a->nactive;
+  for (const DeepLevel& L : a->deep) n += L.nactive;
+  return 1e-6 * n * std::pow((double)a->fb, a->d.q == 9 ? 2 : 3) * (2 * a->d.q + 4) * sizeof(float);
+}
+
 // The interp interface (main-3d.js:3344-3357): the coarse step first (cells
 // under a tile skipped), each tile's ring re-interpolated from the coarse
 // state at t, two substeps in which the ring collides as well, every tile
@@ -659,7 +666,7 @@ int manage(lbm_amr* a) {
 // corrected onto the unrefined side.
 int macro_step_interp(lbm_amr* a) {
   const lbm_amr_desc& d = a->d;
-  int rc = solve_enqueue_covered_step(a->l0, a->block_slot, d.rb, a->G.nbx, a->G.nby);
+  int rc = solve_enqueue_covered_step(a->l0, a->block_slot, d.rb, a->G.nbx, a->G.nby, tiles_mb(a));
   if (rc) return rc;
   const float* ct = solve_lattice(a->l0, 1);  // the state the coarse step read (t)
   float* ct1 = solve_lattice(a->l0, 0);       // the one it wrote (t + 1)
@@ -753,7 +760,7 @@ int macro_step(lbm_amr* a) {
   if (rc0) return rc0;
   HIPCHK(launch_coalesce(d.q, a->pool[0], P0, a->mac_pool, a->G, a->active, a->nactive, a->plan, a->nseam, a->nnear,
                          d.orphans, a->has_body ? &record : nullptr, a->stream));
-  int rc = solve_enqueue_covered_step(a->l0, a->block_slot, d.rb, a->G.nbx, a->G.nby);
+  int rc = solve_enqueue_covered_step(a->l0, a->block_slot, d.rb, a->G.nbx, a->G.nby, tiles_mb(a));
   if (rc) return rc;
   a->step++;
   return LBM_OK;

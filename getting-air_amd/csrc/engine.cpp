@@ -28,6 +28,7 @@
 #include "rigid.h"
 #include "engine.h"
 #include "lattice_pairs.h"
+#include "residency.h"
 
 namespace lbm {
 
@@ -235,6 +236,9 @@ void pair_constants(StepArgs& a, const lbm_desc& d) {
 
 // CHI_EPS of the diffuse coupling (main-3d.js:1026 default 1.5).
 float chi_eps(const lbm_desc& d) { return d.chi_eps > 0.f ? d.chi_eps : 1.5f; }
+
+// Both lattices, MB.
+double lattices_mb(const lbm_solve* s) { return 2e-6 * lattice_elems(s->q, s->N) * s->elem; }
 
 // Force slots: doubles of one step, steps of a launch, and the slots of step
 // `sub` of a launch that read lattice `parity`.
@@ -509,15 +513,17 @@ int flush_force(lbm_solve* s) {
 
 namespace lbm {
 
-int solve_enqueue_covered_step(lbm_solve* s, const int32_t* cover, int rb, int nbx, int nby) {
+int solve_enqueue_covered_step(lbm_solve* s, const int32_t* cover, int rb, int nbx, int nby, double other_mb) {
   const void* fin = s->f[s->parity];
   void* fout = s->f[1 - s->parity];
   StepArgs a = step_args(s, true, false);
+  const bool streamed = s->cached_default && !cache_resident_refined(lattices_mb(s) + 16e-6 * s->N + other_mb);
+  if (streamed) a.swizzle = 0;
   a.cover = cover;
   a.cover_rb = rb;
   a.cover_nbx = nbx;
   a.cover_nby = nby;
-  hipError_t e = launch_step(s->q, s->storage, true, s->nt, s->occ, fin, fout, a, s->bx, s->by, s->stream);
+  hipError_t e = launch_step(s->q, s->storage, true, streamed || s->nt, s->occ, fin, fout, a, s->bx, s->by, s->stream);
   if (e != hipSuccess) return hip_fail(e, "covered step launch");
   s->parity ^= 1;
   s->step++;
@@ -753,21 +759,6 @@ namespace {
 
 const int kTotalsBlocks = 1024;  // max totals partial blocks
 
-// Whether the step's default launches leave both lattices in the 256 MB of
-// last-level cache between steps: ordinary loads and stores, and neighbouring
-// tiles on one XCD, in place of non-temporal access.  us a step before and
-// after, one step a launch: D3Q19 fp32 200x100x19 (60 MB) 13.0 and 10.1,
-// 200x100x78 (240 MB) 44.8 and 34.3, x88 (270 MB) 50.2 and 39.0, x98 (300 MB)
-// 54.9 and 52.1, x115 (350 MB) 63.9 and 65.4; f16 with walls 200x100x157 (240 MB)
-// 50.6 and 43.4; D2Q9 400x5208 (150 MB) 28.4 and 22.3.  Rows of whole 256-cell
-// tiles gain less (256x128x48, 240 MB: 41.8 and 34.7) and small ones nothing
-// (10 MB: f16 5.56 and 5.70; D3Q27 with walls, 60 MB: 12.5 and 13.4).
-bool cache_resident(const lbm_solve* s) {
-  const double mb = 2e-6 * lattice_elems(s->q, s->N) * s->elem;
-  const double least = s->d.nx % 256 ? 0.0 : (s->q == 27 && s->general ? 100.0 : 30.0);
-  return mb >= least && mb <= 270.0;
-}
-
 int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, int by, int flags,
                 lbm_solve** out) {
   if (!out) return fail(LBM_E_INVALID, "null output handle");
@@ -794,7 +785,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
     s->nt = (flags >> 1) & 1;
     s->lin = (flags >> 2) & 1;
     s->occ = (flags >> 4) & 15;
-    if (!arena && !desc->diffuse && cache_resident(s)) {
+    if (!arena && !desc->diffuse && cache_resident(lattices_mb(s), desc->nx, s->q, s->general)) {
       s->nt = 0;
       s->swz = 1;
       s->cached_default = true;

@@ -14,8 +14,9 @@ int hip_fail(hipError_t e, const char* what);
 
 // Hooks the AMR engine uses on its dense L0 solve.
 // One step that skips the cells of refined blocks and writes the
-// macroscopic field of the others.
-int solve_enqueue_covered_step(lbm_solve* s, const int32_t* cover, int rb, int nbx, int nby);
+// macroscopic field of the others.  other_mb: the lattices and fields that the
+// other levels pass through between two such steps.
+int solve_enqueue_covered_step(lbm_solve* s, const int32_t* cover, int rb, int nbx, int nby, double other_mb);
 // which = 0: the lattice holding the current state; 1: the other one.
 float* solve_lattice(lbm_solve* s, int which);
 float* solve_mac(lbm_solve* s);
