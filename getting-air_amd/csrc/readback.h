@@ -5,8 +5,8 @@
 
 namespace lbm {
 
-// Copies `bytes` from the device to pageable host memory behind the work
-// enqueued on `s`, and returns when they have arrived.
+// Copies `bytes` from the device to host memory behind the work enqueued on
+// `s`, and returns when they have arrived.
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t s);
 
 // Copies the `take` most recent of `written` force records (6 doubles each)
