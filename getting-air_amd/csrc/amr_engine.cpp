@@ -871,11 +871,10 @@ int lbm_amr_create(const lbm_amr_desc* desc, lbm_amr** out) {
     l0.sponge_axes[k] = desc->sponge_axes[k];
     l0.sponge_u[k] = desc->sponge_u[k];
   }
-  if ((rc = lbm_solve_create(&l0, &a->l0))) {
+  if ((rc = solve_create_root(&l0, &a->l0))) {
     release(a);
     return rc;
   }
-  solve_no_eager_graphs(a->l0);
   a->stream = solve_stream(a->l0);
   const int rb = desc->rb;
   a->fb = 2 * rb + 2 * kGhost;

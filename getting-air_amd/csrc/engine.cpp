@@ -534,7 +534,6 @@ float* solve_lattice(lbm_solve* s, int which) {
   return static_cast<float*>(s->f[which ? 1 - s->parity : s->parity]);
 }
 float* solve_mac(lbm_solve* s) { return s->mac; }
-void solve_no_eager_graphs(lbm_solve* s) { s->eager_graphs = false; }
 hipStream_t solve_stream(lbm_solve* s) { return s->stream; }
 
 }  // namespace lbm
@@ -759,7 +758,9 @@ namespace {
 
 const int kTotalsBlocks = 1024;  // max totals partial blocks
 
-int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, int by, int flags,
+// `steps`: the solve is stepped by lbm_step (not by the serve loop's or AMR's
+// own launches), so it may take several steps a launch and captures graphs.
+int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, int by, int flags, bool steps,
                 lbm_solve** out) {
   if (!out) return fail(LBM_E_INVALID, "null output handle");
   *out = nullptr;
@@ -768,7 +769,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
   lbm_solve* s = new lbm_solve();
   read_back_retain();
   s->arena = arena;
-  s->eager_graphs = arena == nullptr;
+  s->eager_graphs = steps;
   s->d = *desc;
   s->q = desc->q;
   s->dim = desc->q == 9 ? 2 : 3;
@@ -791,8 +792,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
       s->cached_default = true;
     }
   }
-  // launches of several steps (a pool member's steps are the batched kernel's)
-  if (!arena && !desc->diffuse) {
+  if (steps && !desc->diffuse) {
     s->multi = multi_plan(s->q, desc->nx, desc->ny);
     s->force_subs = s->dim == 2 ? std::max(1, s->multi.steps) : 2;
   }
@@ -834,7 +834,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
       return rc;
     }
   }
-  if (!arena && !desc->diffuse && (rc = build_pair_blocks(s, false))) {
+  if (steps && !desc->diffuse && (rc = build_pair_blocks(s, false))) {
     release(s);
     return rc;
   }
@@ -915,10 +915,14 @@ void default_tile(int storage, int nx, int* bx, int* by, int* flags) {
   *flags = 0x2 | (nx > 0 && nx % 256 == 0 ? 0 : 0x4) | (storage == LBM_STORE_F32 ? 0x60 : 0);
 }
 
+int solve_create_root(const lbm_desc* d, lbm_solve** out) {
+  return create_impl(d, nullptr, nullptr, 0, 0, 0, false, out);
+}
+
 int solve_create_in(const lbm_desc* d, Arena* arena, hipStream_t stream, int bx, int by, int flags,
                     lbm_solve** out) {
   if (!arena || !stream) return fail(LBM_E_INVALID, "pool solve needs an arena and a stream");
-  return create_impl(d, arena, stream, bx, by, flags, out);
+  return create_impl(d, arena, stream, bx, by, flags, false, out);
 }
 
 int solve_batch_entry(lbm_solve* s, BatchSolve* e, uint32_t* ntiles) {
@@ -968,7 +972,7 @@ int lbm_device_info(char* name, size_t name_len, double* hbm_bytes, int32_t* cu_
 
 
 int lbm_solve_create(const lbm_desc* desc, lbm_solve** out) {
-  return create_impl(desc, nullptr, nullptr, 0, 0, 0, out);
+  return create_impl(desc, nullptr, nullptr, 0, 0, 0, true, out);
 }
 
 int lbm_solve_destroy(lbm_solve* s) {
