@@ -746,6 +746,7 @@ int macro_step(lbm_amr* a) {
     force.partials = a->force_partials;
     record.partials = a->force_partials;
     record.steps = 1;
+    record.chunks = 1;
     record.nslots = pool_force_blocks(d.rb, force.nactive);
     record.history = a->history;
     record.written = a->written;

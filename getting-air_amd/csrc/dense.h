@@ -52,14 +52,19 @@ __host__ __device__ inline size_t lat_elem(int q, int i, uint32_t c) {
 
 // Steps a launch takes at most.
 constexpr int kMaxLaunchSteps = 8;
-// Force partials of a launch and where their sums go: slots summed in slot
-// order, one record [fx, fy, fz, tx, ty, tz] per step appended to the history
-// ring.
+// Force partials of a launch and where their sums go: one record [fx, fy, fz,
+// tx, ty, tz] per step appended to the history ring.  Boundary cells' slots are
+// summed in chunks of kForceChunk and the chunks' sums then in their order, the
+// same whichever and however many blocks take them; other slots are one chunk.
+constexpr uint32_t kForceChunk = 1024;
 struct ForceSum {
   const double* partials;       // per slot [3] (force) with `cells`, else [6] (force and torque)
   size_t stride;                // doubles from one step's slots to the next step's
   int32_t steps;                // steps of the launch, kMaxLaunchSteps at most
   uint32_t nslots;
+  uint32_t chunks;
+  double* chunk_sums;           // [chunks][steps][6], with more than one chunk
+  unsigned* arrived;            // blocks that have added theirs (zero between launches)
   const uint32_t* cells;        // per slot its boundary cell, or null
   double centre[3];             // torque arm origin
   int32_t nx, ny, periodic_arm; // 2D: nearest periodic image for the arm
@@ -68,6 +73,8 @@ struct ForceSum {
   unsigned long long* written;  // records written since reset
   uint32_t capacity;
 };
+// Blocks that share the sum, a wave of chunk sums at most.
+__host__ __device__ inline uint32_t force_blocks(const ForceSum& f) { return f.chunks < 64u ? f.chunks : 64u; }
 // Ranks of the boundary cells (ascending cell index) among each 64 cells: a
 // boundary cell's slot is base + the number of mask bits below its own.
 struct BoundaryRank {
@@ -122,9 +129,9 @@ struct StepArgs {
   const BoundaryRank* boundary;  // bounce-back: per 64 cells; null: no force
   const int32_t* force_slot;     // diffuse: per tile; null: no force
   double* force_partials;        // this step's slots (lattice parity buffer)
-  // The previous step's slots are summed by block 0 of this launch (in the
-  // same fixed order as k_force_finalize), so a run of steps needs no separate
-  // reduction launch per step.
+  // The previous launch's slots are summed by the first blocks of this one (in
+  // the same fixed order as k_force_finalize), so a run of steps needs no
+  // separate reduction launch per step.
   int32_t finalize_prev;
   ForceSum prev;
   double body_c[3];           // torque arm origin

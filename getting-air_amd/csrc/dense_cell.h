@@ -13,34 +13,35 @@
 
 namespace lbm {
 
-// Sum of a launch's force slots, step `rec`.  The order is that of 256 lanes
-// whatever the block: lane l takes slots l, l + 256, ... in order, a butterfly
-// folds each 64 lanes, and the four results are added in order.  This is one
-// of the four waves' worth, into out[6] (all 64 lanes of the wave active).
+// Sum of force slots [first, last) of step `rec`.  The order is that of 256
+// lanes whatever the block: lane l takes slots l, l + 256, ... in order, a
+// butterfly folds each 64 lanes, and the four results are added in order.  This
+// is one of the four waves' worth, into out[6] (all 64 lanes of the wave active).
 // With `cells` a slot holds a boundary cell's force alone (3 doubles), and its
 // torque is taken here; otherwise a slot is a tile's force and torque (6
 // doubles).  The slots come from other XCDs' caches, so a wave's time is the
 // latency of its loads: those of two slots are in flight together (more would
 // cost the step kernels this is part of their occupancy).
 template <bool PERIODIC>
-__device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, int part, int lane, double* out) {
+__device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, uint32_t first, uint32_t last, int part,
+                                               int lane, double* out) {
   const double* p = f.partials + (size_t)rec * f.stride;
   double v[6] = {0, 0, 0, 0, 0, 0};
   if (f.cells) {
     constexpr int B = PERIODIC ? 1 : 2;
-    for (uint32_t s0 = part * 64 + lane; s0 < f.nslots; s0 += B * 256) {
+    for (uint32_t s0 = first + part * 64 + lane; s0 < last; s0 += B * 256) {
       uint32_t c[B];
       double F[B][3];
 #pragma unroll
       for (int k = 0; k < B; k++) {
-        const uint32_t s = min(s0 + k * 256, f.nslots - 1);
+        const uint32_t s = min(s0 + k * 256, last - 1);
         c[k] = f.cells[s];
 #pragma unroll
         for (int j = 0; j < 3; j++) F[k][j] = p[(size_t)s * 3 + j];
       }
 #pragma unroll
       for (int k = 0; k < B; k++) {
-        if (k > 0 && s0 + k * 256 >= f.nslots) break;
+        if (k > 0 && s0 + k * 256 >= last) break;
         const uint32_t row = div_invariant(c[k], f.div_nx), z = div_invariant(row, f.div_ny);
         double rx = (double)(c[k] - row * f.nx) - f.centre[0], ry = (double)(row - z * f.ny) - f.centre[1],
                rz = (double)z - f.centre[2];
@@ -59,7 +60,7 @@ __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, int p
       }
     }
   } else {
-    for (uint32_t s = part * 64 + lane; s < f.nslots; s += 256) {
+    for (uint32_t s = first + part * 64 + lane; s < last; s += 256) {
 #pragma unroll
       for (int k = 0; k < 6; k++) v[k] += p[(size_t)s * 6 + k];
     }
@@ -70,23 +71,68 @@ __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, int p
     if (lane == 0) out[k] = t;
   }
 }
-// Appends the records of a launch of up to MAX steps to the history; the whole
-// block (64 threads or more) takes part.
+// Appends the records of a launch of up to MAX steps to the history, or this
+// block's share of it: block `block` of `blocks` sums chunks block, block +
+// blocks, ..., and the last of them to end adds up the chunks.  None waits for
+// another.  The whole block (64 threads or more) takes part.
+// One block alone takes 2 us per 512 slots, which a large body's launches waited
+// for: us a step, one block and shared, D3Q19 120^3 with radius 30 79.4 and 56,
+// 96^3 with 24 35.3 and 26.7, f16 27.2 and 21.2.
 template <bool PERIODIC, int MAX>
-__device__ __forceinline__ void append_force_records(const ForceSum& f) {
-  __shared__ double part[MAX][4][6];
+__device__ __forceinline__ void append_force_records(const ForceSum& f, uint32_t block, uint32_t blocks) {
+  constexpr int ITEMS = MAX * 4 > 16 ? MAX * 4 : 16;
+  __shared__ double part[ITEMS][6];
+  __shared__ bool last_block;
   const int tid = threadIdx.x + threadIdx.y * blockDim.x, waves = (blockDim.x * blockDim.y) >> 6;
   const int n = MAX == 1 ? 1 : f.steps;
-  for (int w = tid >> 6; w < 4 * n; w += waves)
-    sum_force_wave<PERIODIC>(f, w >> 2, w & 3, tid & 63, part[w >> 2][w & 3]);
-  __syncthreads();
-  if (tid < 6 * n) {
-    const int rec = tid / 6, k = tid % 6;
-    const unsigned long long at = *f.written + rec;
-    f.history[(size_t)(at % f.capacity) * 6 + k] = ((part[rec][0][k] + part[rec][1][k]) + part[rec][2][k]) + part[rec][3][k];
+  const bool whole = f.chunks == 1;
+  const uint32_t size = whole ? f.nslots : kForceChunk;
+  const int batch = max(1, waves / (4 * n));  // chunks at a time
+  for (uint32_t c0 = block; c0 < f.chunks; c0 += batch * blocks) {
+    for (int w = tid >> 6; w < batch * 4 * n; w += waves) {
+      const uint32_t c = c0 + (w / (4 * n)) * blocks;
+      if (c >= f.chunks) break;
+      sum_force_wave<PERIODIC>(f, (w >> 2) % n, c * size, min(f.nslots, (c + 1) * size), w & 3, tid & 63, part[w]);
+    }
+    __syncthreads();
+    if (tid < batch * 6 * n && c0 + (tid / (6 * n)) * blocks < f.chunks) {
+      const int q = tid / 6, k = tid - q * 6;
+      const uint32_t c = c0 + (q / n) * blocks;
+      const double v = ((part[q * 4][k] + part[q * 4 + 1][k]) + part[q * 4 + 2][k]) + part[q * 4 + 3][k];
+      if (whole) f.history[(size_t)((*f.written + q % n) % f.capacity) * 6 + k] = v;
+      else __hip_atomic_store(&f.chunk_sums[((size_t)c * n + q % n) * 6 + k], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+  }
+  if (whole) {
+    if (tid == 0) *f.written += n;
+    return;
+  }
+  // The chunk sums are the only data that pass between blocks, written and read
+  // at agent scope past the XCDs' caches, by the first wave (at most 48 lanes);
+  // its wait orders them before the count.  A release and an acquire here would
+  // write back and drop whole caches in the middle of a step (D3Q27 112^3: 63.5
+  // us a step for 60).
+  if (tid == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last_block = __hip_atomic_fetch_add(f.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == blocks - 1;
   }
   __syncthreads();
-  if (tid == 0) *f.written += n;
+  if (!last_block) return;
+  // lane l takes chunks l, l + 64, ... in order, then a butterfly
+  const unsigned long long at = *f.written;
+  for (int w = tid >> 6; w < 6 * n; w += waves) {
+    double v = 0.0;
+    for (uint32_t c = tid & 63; c < f.chunks; c += 64)
+      v += __hip_atomic_load(&f.chunk_sums[(size_t)c * n * 6 + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = wave_sum(v);
+    if ((tid & 63) == 0) f.history[(size_t)((at + w / 6) % f.capacity) * 6 + w % 6] = v;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    *f.arrived = 0u;
+    *f.written = at + n;
+  }
 }
 
 // Slot of a boundary cell: the cells' ascending rank, from a bit mask and a

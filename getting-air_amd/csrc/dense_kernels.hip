@@ -23,8 +23,8 @@ __device__ __forceinline__ T* block_of(T* g, uint32_t c) {
 }
 
 __global__ void __launch_bounds__(512) k_force_finalize(ForceSum a) {
-  if (a.periodic_arm) append_force_records<true, kMaxLaunchSteps>(a);
-  else append_force_records<false, kMaxLaunchSteps>(a);
+  if (a.periodic_arm) append_force_records<true, kMaxLaunchSteps>(a, blockIdx.x, gridDim.x);
+  else append_force_records<false, kMaxLaunchSteps>(a, blockIdx.x, gridDim.x);
 }
 
 template <int Q, class ST>
@@ -247,7 +247,7 @@ hipError_t launch_totals(int q, int storage, const void* f, const TotalsArgs& a,
   return dispatch<OpTotals>(q, storage, f, a, nblocks, s);
 }
 hipError_t launch_force_finalize(const ForceSum& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_force_finalize, dim3(1), dim3(a.steps > 1 ? 512 : 256), 0, s, a);
+  hipLaunchKernelGGL(k_force_finalize, dim3(force_blocks(a)), dim3(a.steps > 1 ? 512 : 256), 0, s, a);
   return hipGetLastError();
 }
 hipError_t launch_classify(const ClassifyArgs& a, hipStream_t s) {

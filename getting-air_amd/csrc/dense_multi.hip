@@ -89,7 +89,7 @@ k_step_multi(const typename ST::T* __restrict__ gin, typename ST::T* __restrict_
     // a block of its own for the previous launch's force records
     if (p.finalize_prev) {
       if (b == 0) {
-        append_force_records<true, kMaxLaunchSteps>(a.prev);
+        append_force_records<true, kMaxLaunchSteps>(a.prev, 0, 1);
         return;
       }
       b--;

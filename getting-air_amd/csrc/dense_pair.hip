@@ -99,7 +99,7 @@ k_step_pair(const float* __restrict__ gin, float* __restrict__ gout, StepArgs a,
     // also steps cells it would hold up all of that block's waves
     if (p.finalize_prev) {
       if (b == 0) {
-        append_force_records<false, 2>(a.prev);
+        append_force_records<false, 2>(a.prev, 0, 1);
         return;
       }
       b--;

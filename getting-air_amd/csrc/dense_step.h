@@ -301,7 +301,8 @@ template <int Q, class ST, bool GEN, bool NT, bool ROW, bool RIGID = false, bool
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Q == 27 ? 6 : 8)))
 k_step(const typename ST::T* __restrict__ gin, typename ST::T* __restrict__ gout, StepArgs a) {
   if constexpr (BODY) {
-    if (a.finalize_prev && blockIdx.x == 0) append_force_records<Q == 9, 1>(a.prev);
+    if (a.finalize_prev && blockIdx.x < force_blocks(a.prev))
+      append_force_records<Q == 9, 1>(a.prev, blockIdx.x, force_blocks(a.prev));
   }
   uint32_t b = blockIdx.x;
   if (a.swizzle) {
@@ -339,7 +340,8 @@ __device__ __forceinline__ void batch_tile(const BatchArgs& B, uint32_t k, int32
   const int p = S.parity ^ (launch & 1);
   const StepArgs& a = *(const StepArgs*)(&sp->args[p]);
   if constexpr (GEN) {
-    if (tile == 0 && (launch > 0 || S.pending) && a.boundary) append_force_records<Q == 9, 1>(a.prev);
+    if (a.boundary && tile < force_blocks(a.prev) && (launch > 0 || S.pending))
+      append_force_records<Q == 9, 1>(a.prev, tile, force_blocks(a.prev));
   }
   // the dither counter of the solve is its step count
   const uint32_t salt = S.step0 + launch;

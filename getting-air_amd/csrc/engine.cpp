@@ -240,6 +240,9 @@ float chi_eps(const lbm_desc& d) { return d.chi_eps > 0.f ? d.chi_eps : 1.5f; }
 // Both lattices, MB.
 double lattices_mb(const lbm_solve* s) { return 2e-6 * lattice_elems(s->q, s->N) * s->elem; }
 
+// Chunks of the boundary cells' sum, one at least.
+uint32_t force_chunks(size_t cells) { return (uint32_t)std::max<size_t>(1, (cells + kForceChunk - 1) / kForceChunk); }
+
 // Force slots: doubles of one step, steps of a launch, and the slots of step
 // `sub` of a launch that read lattice `parity`.
 size_t force_stride(const lbm_solve* s) { return (size_t)s->nslots * (s->d.diffuse ? 6 : 3); }
@@ -253,6 +256,9 @@ ForceSum force_sum(const lbm_solve* s, int parity, int steps) {
   f.stride = force_stride(s);
   f.steps = steps;
   f.nslots = s->nslots;
+  f.chunks = s->d.diffuse ? 1 : force_chunks(s->nslots);
+  f.chunk_sums = force_set(s, 2, 0);  // past both parities' slots
+  f.arrived = s->counters + 2;
   f.cells = s->d.diffuse ? nullptr : s->boundary_cells;
   f.centre[0] = s->d.body.centre[0];
   f.centre[1] = s->d.body.centre[1];
@@ -340,8 +346,8 @@ int build_boundary_slots(lbm_solve* s) {
   }
   s->rank_bytes = groups * sizeof(BoundaryRank);
   s->cell_bytes = std::max<size_t>(n, 1) * 4;
-  // one set per lattice parity and step of a launch
-  s->partial_bytes = (size_t)2 * s->force_subs * std::max<size_t>(n, 1) * 3 * 8;
+  // one set per lattice parity and step of a launch, then the chunks' sums
+  s->partial_bytes = (size_t)s->force_subs * (2 * std::max<size_t>(n, 1) * 3 + force_chunks(n) * 6) * 8;
   int rc = dalloc(s, &s->ranks, s->rank_bytes);
   if (!rc) rc = dalloc(s, &s->boundary_cells, s->cell_bytes);
   if (!rc) rc = dalloc(s, &s->force_partials, s->partial_bytes);
@@ -883,7 +889,7 @@ size_t solve_footprint(const lbm_desc* d) {
                  al((size_t)kHistoryCap * 6 * 8) + al(8) + al(64) + al(8);
   if (d->body.shape != LBM_BODY_NONE) {
     // class bytes, link masks; the boundary cells' ranks, indices and two
-    // parity sets of 3 partials.  A boundary cell's centre lies less than a
+    // parity sets of 3 partials, and the chunks' sums.  A boundary cell's centre lies less than a
     // link from the surface (sqrt 3, in 2D sqrt 2), so the unit cells around
     // them lie in that shell grown by half a cell's diagonal, whose volume
     // bounds their number; and never less than a slot index per tile of 64
@@ -895,7 +901,8 @@ size_t solve_footprint(const lbm_desc* d) {
     const size_t cells = (size_t)std::min((double)n, shell + 1.0);
     const size_t tiles = (n + 63) / 64 + d->ny * (d->q == 9 ? 1 : d->nz);
     total += al(n) + al(n * 4) +
-             std::max(al((n + 63) / 64 * sizeof(BoundaryRank)) + al(cells * 4) + al(2 * cells * 3 * 8),
+             std::max(al((n + 63) / 64 * sizeof(BoundaryRank)) + al(cells * 4) +
+                          al((2 * cells * 3 + force_chunks(cells) * 6) * 8),
                       al(tiles * 4) + al(2 * tiles * 6 * 8));
   }
   return total;
