@@ -792,7 +792,7 @@ int create_impl(const lbm_desc* desc, Arena* arena, hipStream_t stream, int bx, 
     s->nt = (flags >> 1) & 1;
     s->lin = (flags >> 2) & 1;
     s->occ = (flags >> 4) & 15;
-    if (!arena && !desc->diffuse && cache_resident(lattices_mb(s), desc->nx, s->q, s->general)) {
+    if (!arena && !desc->diffuse && cache_resident(lattices_mb(s), s->N, desc->nx, s->q, (int)s->elem, s->general, s->body)) {
       s->nt = 0;
       s->swz = 1;
       s->cached_default = true;

@@ -12,12 +12,27 @@ SRC = r"""
 static double refined(int q, double cells, int tile, double tiles) {
   return 1e-6 * (cells + tiles * tile) * (2 * q + 4) * 4;
 }
+static bool dense(int q, int nx, int ny, int nz, int elem, bool general, bool body) {
+  const double n = (double)nx * ny * nz;
+  return lbm::cache_resident(2e-6 * n * q * elem, n, nx, q, elem, general, body);
+}
 int main() {
   using namespace lbm;
+  // a body, fp32 and f16; 2D; walls
+  printf("%d%d%d%d%d%d%d%d ", dense(19, 64, 64, 64, 4, true, true), dense(19, 128, 70, 37, 4, true, true),
+         dense(19, 72, 72, 72, 4, true, true), dense(19, 96, 96, 96, 4, true, true), dense(27, 64, 64, 64, 4, true, true),
+         dense(27, 96, 64, 64, 4, true, true), dense(27, 80, 80, 80, 4, true, true), dense(27, 48, 48, 48, 4, true, true));
+  printf("%d%d%d%d%d%d%d%d ", dense(19, 64, 64, 64, 2, true, true), dense(19, 128, 64, 64, 2, true, true),
+         dense(19, 80, 80, 80, 2, true, true), dense(19, 100, 100, 100, 2, true, true), dense(27, 64, 64, 64, 2, true, true),
+         dense(27, 128, 64, 64, 2, true, true), dense(27, 80, 80, 80, 2, true, true), dense(27, 100, 100, 100, 2, true, true));
+  printf("%d%d%d %d%d%d%d ", dense(9, 768, 768, 1, 4, true, true), dense(9, 1024, 1024, 1, 2, true, true),
+         dense(9, 1440, 1440, 1, 4, true, true), dense(19, 64, 64, 64, 4, true, false), dense(19, 72, 72, 72, 4, true, false),
+         dense(19, 64, 64, 64, 2, true, false), dense(19, 64, 64, 64, 4, false, false));
   const int t3 = 20 * 20 * 20, t2 = 20 * 20, n96 = 96 * 96 * 96, n80 = 80 * 80 * 80, n2 = 1024 * 1024;
   printf("%d%d%d%d%d %d%d%d%d%d%d\n",
-         cache_resident(60, 200, 19, false), cache_resident(270, 200, 19, true), cache_resident(350, 200, 19, false),
-         cache_resident(10, 256, 19, false), cache_resident(60, 256, 27, true),
+         cache_resident(60, 0.4e6, 200, 19, 4, false, false), cache_resident(270, 1.8e6, 200, 19, 4, true, false),
+         cache_resident(350, 2.3e6, 200, 19, 4, false, false), cache_resident(10, 0.13e6, 256, 19, 2, false, false),
+         cache_resident(60, 0.28e6, 256, 27, 4, true, false),
          cache_resident_refined(refined(27, n96, t3, 17)), cache_resident_refined(refined(27, n96, t3, 69)),
          cache_resident_refined(refined(27, n80, t3, 60)), cache_resident_refined(refined(27, n80, t3, 100)),
          cache_resident_refined(refined(9, n2, t2, 4096)), cache_resident_refined(refined(9, n2, t2, 6553)));
@@ -31,4 +46,4 @@ def test_rules_lie_between_the_measured_sides(tmp_path):
     exe = str(tmp_path / "r")
     subprocess.check_call(["g++", "-std=c++17", "-I", os.path.join(ROOT, "getting-air_amd", "csrc"), str(src), "-o", exe])
     # measured faster in the cache (1) or streamed (0)
-    assert subprocess.check_output([exe], text=True).split() == ["11000", "101010"]
+    assert subprocess.check_output([exe], text=True).split() == ["00110011", "10010001", "001", "0101", "11000", "101010"]
