@@ -439,18 +439,24 @@ PairPlan pair_plan(int q, int storage, bool general, int nx, int ny, int nz, con
     std::fill(chunks.begin(), chunks.end(), 1);
     best = (nz + 2.0) * cols / cus;
   }
-  // Pairs where their estimate is the shorter one.  A pair takes the longest
-  // block's planes at a plane's latency, or the traffic at the rate it reaches;
-  // planes that are not whole layout blocks cost address arithmetic.  Fitted to
-  // 18 grids from 32^3 to 240^3 (us; for example D3Q19 96^3 49.8 one by one,
-  // 35.5 in pairs; 64x32x32 7.5 and 9.2).
-  const bool whole = (uint64_t)nx * ny % kLatBlock == 0;
-  const double plane_us = q == 19 ? (general ? 5.2 : 3.5) : (general ? 7.2 : 4.8);
-  const double pair_us = std::max(plane_us * best, bytes * 1.07 / 4.7e6 * (q == 19 ? 1.0 : 1.2)) * (whole ? 1.0 : 1.25);
-  // one by one, lattices that stay in the last-level cache or not
-  const double step_us = std::max(3.8, bytes <= 270e6 ? bytes / 7.2e6 + 2.0
-                                                      : (bytes / 6.0e6 + 2.0) * (nx % (int)kLatBlock == 0 ? 1.0 : 1.1));
-  if (!always && pair_us > 0.97 * 2.0 * step_us) return plan;
+  // Pairs where their estimate is the shorter one: a pair takes the longest
+  // block's planes at a plane's latency and the traffic at the rate it reaches,
+  // less where planes are not whole layout blocks (address arithmetic) or rows
+  // are not (split lines); a one-step launch the traffic, at the rate of the
+  // last-level cache as long as both lattices fit it.  Fitted to 51 grids from
+  // 32^3 to 240^3 of either lattice, each periodic, with walls and with a body:
+  // the form chosen is 0.3% off the faster one on average, 14% at most.  us a
+  // step, one by one and in pairs: D3Q19 96^3 20.6 and 17.9, 100^3 23.0 and 27.6,
+  // 64x32x32 3.6 and 4.5, 140^3 with a body 78.0 and 82.8, 160^3 107 and 83;
+  // D3Q27 with walls 190x99x99 80 and 64, 150x75x50 22.7 and 26.0.
+  const bool whole = (uint64_t)nx * ny % kLatBlock == 0, row = nx % (int)kLatBlock == 0, body = !boundary.empty();
+  const double mb = 1e-6 * bytes;
+  const double plane_us = (general ? (q == 19 ? 2.9 : 3.3) : 2.1) + (whole ? 0.0 : 0.8);
+  const double mb_us = (row ? 0.15 : 0.165) - (general && q == 27 ? 0.03 : 0.0) + (body ? 0.02 : 0.0);
+  const double pair_us = plane_us * best + mb_us * mb;
+  const double step_us = std::max(3.8, mb <= 270.0 ? mb / 7.1 + (body ? 6.0 : (general ? 3.0 : 2.0))
+                                                   : mb / (row ? 6.0 : 5.4) + 2.0);
+  if (!always && pair_us > 2.0 * step_us) return plan;
   plan.rows = rows;
   // chunk by chunk over the columns, so that neighbouring columns march the
   // same planes at the same time on one XCD

@@ -82,7 +82,7 @@ def test_bodies(q, grid, body, solid_eq):
 
 # grids that the engine's choice sends to pairs
 @pytest.mark.parametrize("q,grid,extra", [
-    (19, (122, 122, 122), {}), (19, (100, 100, 100), FORCE), (27, (100, 100, 150), {}), (27, (190, 99, 99), FORCE),
+    (19, (122, 122, 122), {}), (19, (190, 99, 99), FORCE), (27, (100, 100, 150), {}), (27, (190, 99, 99), FORCE),
     (27, (255, 129, 130), {"walls": [0, 1, 1], "wallU": [0.01, -0.02]}),
     (27, (255, 130, 130), dict(FORCE, walls=[1, 1, 0])), (19, (256, 128, 64), {"walls": [0, 1, 0]})])
 def test_chosen_pairs(q, grid, extra):
