@@ -835,7 +835,7 @@ k_coalesce(const float* __restrict__ gp, ParentRef P, const float* __restrict__ 
     coalesce_mac<Q, RB, PP>(P, mac_pool, G, active, nactive, b);
     return;
   }
-  if constexpr (!PP && Lattice<Q>::D == 3) append_force_records<false, 1>(force, 0, 1);
+  if constexpr (!PP && Lattice<Q>::D == 3) append_force_records<false, 1, false>(force, 0, 1);
 }
 
 // ---------------------------------------------------------------------------

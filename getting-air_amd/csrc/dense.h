@@ -133,7 +133,6 @@ struct StepArgs {
   // the same fixed order as k_force_finalize), so a run of steps needs no
   // separate reduction launch per step.
   int32_t finalize_prev;
-  ForceSum prev;
   double body_c[3];           // torque arm origin
   int32_t periodic_arm;       // 2D: nearest periodic image for the arm
   // The diffuse penalty coupling of the pinned body (the DIFF kernels, in
@@ -156,6 +155,7 @@ struct StepArgs {
   // alternate with the lattice parity, so graph replays keep counting).
   const uint32_t* salt_in;
   uint32_t* salt_out;
+  ForceSum prev;       // finalize_prev's
 };
 
 // The serve loop's batched step: per-solve state in device memory.

@@ -22,12 +22,12 @@ namespace lbm {
 // doubles).  The slots come from other XCDs' caches, so a wave's time is the
 // latency of its loads: those of two slots are in flight together (more would
 // cost the step kernels this is part of their occupancy).
-template <bool PERIODIC>
+template <bool PERIODIC, bool CELLS>
 __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, uint32_t first, uint32_t last, int part,
                                                int lane, double* out) {
   const double* p = f.partials + (size_t)rec * f.stride;
   double v[6] = {0, 0, 0, 0, 0, 0};
-  if (f.cells) {
+  if (CELLS && f.cells) {
     constexpr int B = PERIODIC ? 1 : 2;
     for (uint32_t s0 = first + part * 64 + lane; s0 < last; s0 += B * 256) {
       uint32_t c[B];
@@ -78,24 +78,25 @@ __device__ __forceinline__ void sum_force_wave(const ForceSum& f, int rec, uint3
 // One block alone takes 2 us per 512 slots, which a large body's launches waited
 // for: us a step, one block and shared, D3Q19 120^3 with radius 30 79.4 and 56,
 // 96^3 with 24 35.3 and 26.7, f16 27.2 and 21.2.
-template <bool PERIODIC, int MAX>
+// CELLS false: f holds no boundary cells, one chunk.
+template <bool PERIODIC, int MAX, bool CELLS = true>
 __device__ __forceinline__ void append_force_records(const ForceSum& f, uint32_t block, uint32_t blocks) {
   constexpr int ITEMS = MAX * 4 > 16 ? MAX * 4 : 16;
   __shared__ double part[ITEMS][6];
   __shared__ bool last_block;
   const int tid = threadIdx.x + threadIdx.y * blockDim.x, waves = (blockDim.x * blockDim.y) >> 6;
   const int n = MAX == 1 ? 1 : f.steps;
-  const bool whole = f.chunks == 1;
+  const bool whole = !CELLS || f.chunks == 1;
   const uint32_t size = whole ? f.nslots : kForceChunk;
   const int batch = max(1, waves / (4 * n));  // chunks at a time
-  for (uint32_t c0 = block; c0 < f.chunks; c0 += batch * blocks) {
+  for (uint32_t c0 = block; c0 < (CELLS ? f.chunks : 1u); c0 += batch * blocks) {
     for (int w = tid >> 6; w < batch * 4 * n; w += waves) {
       const uint32_t c = c0 + (w / (4 * n)) * blocks;
-      if (c >= f.chunks) break;
-      sum_force_wave<PERIODIC>(f, (w >> 2) % n, c * size, min(f.nslots, (c + 1) * size), w & 3, tid & 63, part[w]);
+      if (c >= (CELLS ? f.chunks : 1u)) break;
+      sum_force_wave<PERIODIC, CELLS>(f, (w >> 2) % n, c * size, min(f.nslots, (c + 1) * size), w & 3, tid & 63, part[w]);
     }
     __syncthreads();
-    if (tid < batch * 6 * n && c0 + (tid / (6 * n)) * blocks < f.chunks) {
+    if (tid < batch * 6 * n && c0 + (tid / (6 * n)) * blocks < (CELLS ? f.chunks : 1u)) {
       const int q = tid / 6, k = tid - q * 6;
       const uint32_t c = c0 + (q / n) * blocks;
       const double v = ((part[q * 4][k] + part[q * 4 + 1][k]) + part[q * 4 + 2][k]) + part[q * 4 + 3][k];
