@@ -38,6 +38,7 @@
 // 83-93 us: their frames are read and computed too often.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <vector>
 #include "dense.h"
@@ -492,10 +493,17 @@ static hipError_t run_pair(bool general, const float* fin, float* fout, const St
   hipError_t err = hipSuccess;
   auto go = [&](auto G, auto F, auto A) {
     constexpr auto k = k_step_pair<Q, decltype(G)::value, decltype(F)::value, decltype(A)::value>;
-    // gfx950 has 160 KiB of LDS per CU; a launch above 64 KiB asks for it
-    static const hipError_t grown =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if ((err = grown) != hipSuccess) return;
+    // gfx950 has 160 KiB of LDS per CU; a launch above 64 KiB asks for it, once
+    // on each GPU
+    static std::atomic<uint64_t> grown{0};
+    int dev = 0;
+    if ((err = hipGetDevice(&dev)) != hipSuccess) return;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(grown.load() & bit)) {
+      err = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (err != hipSuccess) return;
+      grown.fetch_or(bit);
+    }
     hipLaunchKernelGGL(k, dim3(p.nblocks + (p.finalize_prev ? 1 : 0)), dim3(64 * (p.rows + 3)), lds, s, fin, fout, a, p);
     err = hipGetLastError();
   };
