@@ -1,5 +1,5 @@
 // One cell of the dense step, shared by the one-step kernels
-// (dense_kernels.hip) and the multi-step ones (dense_pair.hip): halfway
+// (dense_step.h) and the multi-step ones (dense_pair.hip, dense_multi.hip): halfway
 // bounce-back with the momentum it exchanges, the sponge weight, and the
 // BGK/TRT relaxation in pair form.  Every kernel runs the same arithmetic
 // here, so a step's result does not depend on which of them took it.

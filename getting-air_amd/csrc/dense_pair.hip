@@ -30,11 +30,11 @@
 //
 // Measured (MI355X, us per step, one by one -> in pairs): D3Q19 256x128x128
 // periodic 106.0 -> 70.8, with the sphere and sponge 105.9 -> 76.0; 256^3 436
-// -> 259; D3Q27 128^3 77.4 -> 58.9.  At 256x128x128 a pair reads 361 MB and
-// writes 319 MB (1.13 and 1.00 times the lattice); it is bound by the block's
-// own latency (load, barrier, LDS, store of a plane: 4.4 us a plane with 40
-// blocks on the chip, 5.9 with 240) rather than by HBM or its VALU (a third
-// busy).  Smaller columns (4 to 6 rows, two blocks per CU) measured slower,
+// -> 259; D3Q27 128^3 77.4 -> 58.9.  At 256x128x128 a pair reads 370 MB (with
+// the sphere 406) and writes 322 MB, 1.16 (1.28) and 1.01 times the lattice; it
+// is bound by the block's own latency (load, barrier, LDS, store of a plane: 4.4
+// us a plane with 40 blocks on the chip, 6.2 with 240) rather than by HBM (three
+// quarters of a copy's rate) or its VALU (under half busy).  Smaller columns (4 to 6 rows, two blocks per CU) measured slower,
 // 83-93 us: their frames are read and computed too often.
 #include <hip/hip_runtime.h>
 #include <algorithm>

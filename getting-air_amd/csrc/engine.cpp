@@ -1,14 +1,14 @@
 // Host side of the dense engine: the lbm_solve object behind include/lbm.h.
 //
 // A solve owns two population lattices (ping-pong, shifted storage), the
-// macroscopic field, the body classification, the per-tile force slots and
-// one HIP stream.  Each step is one fused stream-collide launch (which also
-// reduces the momentum-exchange force of the tiles touching the body into
-// FP64 slots) followed, when a body is present, by a one-wave launch that
-// sums the slots in a fixed order into the force history.  Only the last step
-// of an lbm_step(n) call writes the macroscopic field, which is what the
-// reference's readbacks observe (main-3d.js:3506-3539).  Chunks of steps are
-// replayed from captured hipGraphs.
+// macroscopic field, the body classification, the force slots (one per
+// boundary cell) and one HIP stream.  A launch advances one step or several
+// (launch_steps) and leaves the momentum exchange of each boundary cell and step
+// in its FP64 slot; the next launch, or a launch of its own after the last, sums
+// the slots in a fixed order into the force history.  Only the last step of an
+// lbm_step(n) call writes the macroscopic field, which is what the reference's
+// readbacks observe (main-3d.js:3506-3539).  Chunks of launches are replayed
+// from captured hipGraphs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1345,11 +1345,8 @@ int lbm_set_launch_steps(lbm_solve* s, int32_t steps) {
   }
   HIPCHK(hipStreamSynchronize(s->stream));
   drop_graphs(s);
-  if (s->pair_blocks) {
-    HIPCHK(hipFree(s->pair_blocks));
-    s->pair_blocks = nullptr;
-    s->bytes -= (size_t)s->pair_nblocks * sizeof(PairBlock);
-  }
+  dfree(s, s->pair_blocks, (size_t)s->pair_nblocks * sizeof(PairBlock));
+  s->pair_blocks = nullptr;
   s->pair_rows = 0;
   s->multi = MultiPlan{};
   if (s->dim == 2 && steps != 1) {
