@@ -300,9 +300,11 @@ template <int Q, class ST, bool GEN, bool NT, bool ROW, bool RIGID = false, bool
           bool BODY = GEN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Q == 27 ? 6 : 8)))
 k_step(const typename ST::T* __restrict__ gin, typename ST::T* __restrict__ gout, StepArgs a) {
-  if constexpr (BODY) {
-    if (a.finalize_prev && blockIdx.x < force_blocks(a.prev))
-      append_force_records<Q == 9, 1>(a.prev, blockIdx.x, force_blocks(a.prev));
+  // a moving body's records are k_rigid_force's; the diffuse coupling's slots
+  // are one chunk
+  if constexpr (BODY && !RIGID) {
+    if (a.finalize_prev && blockIdx.x < (DIFF ? 1u : force_blocks(a.prev)))
+      append_force_records<Q == 9, 1, !DIFF>(a.prev, blockIdx.x, DIFF ? 1u : force_blocks(a.prev));
   }
   uint32_t b = blockIdx.x;
   if (a.swizzle) {
