@@ -15,9 +15,9 @@ namespace lbm {
 //
 // Grids of about as many bytes as the XCDs' own caches hold are an exception
 // where a few blocks are slow, those next to a body and, in rows of whole
-// layout blocks, to walls: ordinary stores wait in those caches for the end of
-// the launch, behind the slow blocks.  Ordinary over non-temporal, two sizes of
-// body: D3Q19 fp32 64^3 1.18, 1.08, 128x70x37 1.11, 1.02, 96^3 0.91, 0.91;
+// layout blocks, to walls.  Measured, not explained: ordinary loads with
+// non-temporal stores are slower than both there (64^3 1.2 times), so neither
+// alone is it.  Ordinary over non-temporal, two sizes of body: D3Q19 fp32 64^3 1.18, 1.08, 128x70x37 1.11, 1.02, 96^3 0.91, 0.91;
 // D3Q27 56^3 1.02, 1.07, 64^3 1.40, 1.25, 96x64x64 1.11, 1.03, 80^3 0.95, 0.84;
 // f16 D3Q19 64^3 0.99, 0.94, 128x64x64 1.18, 1.17, 80^3 1.12, 1.14, 100^3 0.97,
 // 0.94; D3Q27 64^3 1.13, 1.12, 128x64x64 1.22, 1.18, 80^3 1.12, 1.09, 100^3
